@@ -232,6 +232,30 @@ __device__ __forceinline__ f32x16 mfma_f16_32x32x16(f16x8 a, f16x8 b, f32x16 c) 
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
+// Block sums to fp32 without v_cvt_f32_i32, which issues at less than half the
+// rate of an fp32 subtraction: the int8 MFMA starts from the bits of a float
+// in the middle of its binade, 1/(2 pi) = 0x3e22f983 (one ulp is 2^-26 and
+// integer sums from -2292099 to 6096508 stay in the binade; it is also an
+// inline constant, so the MFMA's C operand takes no registers), and
+// subtracting that float from the result leaves S * 2^-26 exactly. A 16 * S_b
+// of a 32-element block is at most 16 * 32 * 8 * 128 = 524288 in magnitude.
+// 32x32x32 block sums scaled and added in registers (two waves per SIMD):
+// 68.4 ns an item with the conversion, 50.2 with the subtraction, 48.4 with
+// neither; whole products: 2048x11008x4096 262.9 -> 258.1 us, 480x1536x4096
+// 17.6 -> 16.9. The whole-K tiles (6.98 against 7.00 us) and the tile GEMVs
+// (2 % either way) gain nothing from it and keep the conversion.
+constexpr int32_t kSumBase = 0x3e22f983;
+__device__ __forceinline__ i32x16 sum_base16() {
+    i32x16 v;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = kSumBase;
+    return v;
+}
+// S * 2^-26 of an MFMA result r = kSumBase + S
+__device__ __forceinline__ float based_sum(int32_t r) { return f32_from((uint32_t)r) - f32_from((uint32_t)kSumBase); }
+// C from the scaled sum of 16 * S_b * 2^-26 * d terms
+constexpr float kBasedSumScale = 0x1p+22f;
+
 // q4_K scale and min of sub-block j (0..7) from the 12 packed bytes (hd[1..3];
 // hd[0] holds d and dmin), with the reference's decode
 // (llama_reference.cpp:116-121).
