@@ -1,0 +1,86 @@
+"""Device weight quantizers at the edges of their layout and arithmetic, byte
+for byte against the oracle: block counts around the 64 blocks (8 super-blocks)
+of a workgroup, q4_0 outputs two bytes off a dword, and the values whose
+quotient the q4_K kernel forms by correction steps: quantization ties, ranges
+on both sides of the bounds [2^-40, 2^40] of those steps, ranges far below the
+offset, infinities and NaN."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from test_gpu_exact import dev, say
+
+pytestmark = pytest.mark.gpu
+
+
+def expected(oracle, qtype, x):
+    y = oracle.quantize_q4_0(x) if qtype == 0 else oracle.quantize_q4_K(x)
+    return y.view(np.uint8).reshape(-1)
+
+
+@pytest.mark.parametrize("qtype,rows,k", [(0, 1, 32), (0, 63, 32), (0, 65, 32), (0, 255, 32), (0, 257, 96),
+                                          (1, 1, 256), (1, 7, 256), (1, 9, 256), (1, 31, 256), (1, 33, 768)])
+@pytest.mark.parametrize("offset", [0, 2])
+def test_block_counts(hip, torch_gpu, oracle, qtype, rows, k, offset):
+    torch = torch_gpu
+    if qtype == 1 and offset:
+        pytest.skip("q4_K outputs are 16-byte aligned")
+    say(f"weight quantizer type={qtype} rows={rows} k={k} offset={offset}")
+    x = np.random.default_rng(rows + k).standard_normal((rows, k)).astype(np.float32)
+    expect = expected(oracle, qtype, x)
+    buf = torch.full((expect.size + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+    hip.quantize_weights_gpu(qtype, dev(torch, x), out=buf[16 + offset:16 + offset + expect.size])
+    torch.cuda.synchronize()
+    got = buf.cpu().numpy()
+    assert np.array_equal(got[16 + offset:16 + offset + expect.size], expect)
+    assert (np.delete(got, np.s_[16 + offset:16 + offset + expect.size]) == 0xA5).all()
+
+
+def value_rows(k):
+    rng = np.random.default_rng(7)
+    rows = []
+    for step in (1.0, 0.1, 3.0, 1 / 3, 0.7, 1e-3):  # multiples of half a step: ties of x / ls + lm
+        rows.append(np.float32(step) * rng.integers(-31, 32, k).astype(np.float32) / 2)
+        rows.append(np.float32(step) * (rng.integers(0, 31, k).astype(np.float32) / 2 - np.float32(5.3)))
+    for e in (-148, -126, -100, -45, -41, -40, -39, -37, 35, 36, 37, 40, 44, 100, 126):
+        rows.append((rng.uniform(-1, 1, k) * 2.0 ** e).astype(np.float32))
+    for base in (1.0, -3.0, 1e6, -1e-20, 1e30):  # ranges of a few units in the last place
+        rows.append(np.float32(base) * (1 + rng.integers(0, 20, k).astype(np.float32) * np.float32(2.0 ** -23)))
+    wide = rng.standard_normal(k).astype(np.float32)
+    wide[::7] *= np.float32(1e-30)
+    rows.append(wide)
+    return np.ascontiguousarray(np.stack(rows).astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype", [0, 1])
+def test_values(hip, torch_gpu, oracle, qtype):
+    torch = torch_gpu
+    say(f"weight quantizer values type={qtype}")
+    x = value_rows(4096)
+    got = hip.quantize_weights_gpu(qtype, dev(torch, x)).cpu().numpy()
+    expect = expected(oracle, qtype, x).reshape(x.shape[0], -1)
+    differs = (got != expect).any(1)
+    if qtype == 0:
+        # where a scale max / -8 is below 2^-128 its reciprocal overflows, and the
+        # conversion of the infinite product to int is the device's, not x86's
+        differs &= np.abs(x).reshape(x.shape[0], -1, 32).max(2).min(1) >= 2.0 ** -125
+    bad = np.flatnonzero(differs)
+    assert bad.size == 0, f"rows {bad} differ"
+
+
+def test_q4_K_infinite_and_nan(hip, torch_gpu, oracle):
+    """A super-block with an infinite value (its range, and so every quotient,
+    leaves the correction steps' bounds) or a NaN beside finite values."""
+    torch = torch_gpu
+    say("q4_K inf / nan")
+    x = np.random.default_rng(3).standard_normal((4, 512)).astype(np.float32)
+    x[0, 40] = np.inf
+    x[1, 300] = -np.inf
+    x[2, 33] = np.nan
+    got = hip.quantize_weights_gpu(1, dev(torch, x)).cpu().numpy()
+    expect = expected(oracle, 1, x).reshape(4, -1)
+    # the packed scales of a super-block whose scale is infinite or NaN come
+    # from float -> int conversions of NaN; compare the finite super-blocks
+    for r, b in [(0, 1), (1, 0), (3, 0), (3, 1), (2, 1)]:
+        assert np.array_equal(got[r, 144 * b:144 * b + 144], expect[r, 144 * b:144 * b + 144]), (r, b)
