@@ -68,7 +68,10 @@ typedef enum {
                             m = 3..6 by format and k (iq2_xxs at k == 4096 from
                             m = 9, m = 5..8 a tile with two-half copies) */
     PFNG_PATH_MFMA = 2,  /* int8-MFMA GEMM, LDS-staged tiles: q4_0 with k % 128 == 0,
-                            q4_K and iq2_xxs for every k % 256 == 0; k <= 2^24 */
+                            q4_K and iq2_xxs for every k % 256 == 0; k <= 2^24.
+                            Small m of the K-quants (up to 64, from k = 2048 up to
+                            128) run on the GEMV's 16-row tiles at the k that
+                            PFNG_PATH_GEMV declines for them */
     PFNG_PATH_NAIVE = 3  /* one thread per output, the reference's exact fp32 order */
 } pfng_path;
 
@@ -179,7 +182,9 @@ int pfng_hip_compute_noalloc(int type, const float *activation, const void *weig
  *   iq2_xxs: out[(m*n + n)*(k/256) + b]    = sum_j (2 s_j + 1) * S_j
  * Where PFNG_PATH_MFMA runs q4_K on whole-K tiles (k = 1024 or 1536), which
  * split super-blocks between K slices and join the parts only in fp32, the
- * sums come from the 64 x 64 two-slice tiles that shape would otherwise take.
+ * sums come from the 64 x 64 two-slice tiles that shape would otherwise take,
+ * as they do where it runs a K-quant on 16-row tiles (small m at the k that
+ * PFNG_PATH_GEMV does not take there).
  * For verification at small sizes; not a performance path. */
 int pfng_hip_block_isums(int type, const void *weight, const void *act_q, int32_t *out, int64_t m, int64_t n,
                          int64_t k, void *stream);

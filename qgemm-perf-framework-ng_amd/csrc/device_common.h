@@ -404,9 +404,11 @@ __device__ __forceinline__ void run_copy(const uint8_t *src, uint32_t rstride, i
 // the kN % 64 == 16 chunks left by one 4-byte copy (lane l: dword l % 4 of
 // chunk kN / 64 * 64 + l / 4), so exactly kN * 16 bytes are written, every
 // lane active, and in as many instructions as run_copy issues.
-template <int kRows, int kCols>
+// kParity: row r starts 2 bytes earlier where first + r * odd is odd (src is
+// 2 bytes before the later of the two starts).
+template <int kRows, int kCols, bool kParity = false>
 __device__ __forceinline__ void run_copy_exact(const uint8_t *src, uint32_t rstride, int col0, int rvalid,
-                                               uint8_t *dst, int lane) {
+                                               uint8_t *dst, int lane, int odd = 0, int first = 0) {
     constexpr int kN = kRows * kCols, kFull = kN / 64;
     static_assert(kN % 64 == 16, "a 16-chunk tail: one 4-byte copy of 64 lanes");
 #pragma unroll
@@ -415,7 +417,8 @@ __device__ __forceinline__ void run_copy_exact(const uint8_t *src, uint32_t rstr
         int r = p / kCols;
         const int col = col0 + p - r * kCols;
         if (r > rvalid - 1) r = rvalid - 1;
-        const uint32_t off = (uint32_t)r * rstride + 16u * (uint32_t)col;
+        uint32_t off = (uint32_t)r * rstride + 16u * (uint32_t)col;
+        if constexpr (kParity) off += 2u - 2u * (uint32_t)((first + r * odd) & 1);
         __builtin_amdgcn_global_load_lds(src + off, (__attribute__((address_space(3))) void *)(dst + i * 1024), 16,
                                          0, 0);
     }
@@ -423,7 +426,8 @@ __device__ __forceinline__ void run_copy_exact(const uint8_t *src, uint32_t rstr
     int r = p / kCols;
     const int col = col0 + p - r * kCols;
     if (r > rvalid - 1) r = rvalid - 1;
-    const uint32_t off = (uint32_t)r * rstride + 16u * (uint32_t)col + 4u * (uint32_t)(lane & 3);
+    uint32_t off = (uint32_t)r * rstride + 16u * (uint32_t)col + 4u * (uint32_t)(lane & 3);
+    if constexpr (kParity) off += 2u - 2u * (uint32_t)((first + r * odd) & 1);
     __builtin_amdgcn_global_load_lds(src + off, (__attribute__((address_space(3))) void *)(dst + kFull * 1024), 4, 0,
                                      0);
 }

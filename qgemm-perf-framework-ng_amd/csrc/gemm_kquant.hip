@@ -733,7 +733,7 @@ using KqBigS2 = KqConfig<T, 128, 64, 2, 2, 1, 2>;
 template <Kq T>
 using KqSmallS2 = KqConfig<T, 64, 64, 2, 2, 1, 2>;
 
-enum { kCfgBig = 0, kCfgTiny = 2, kCfgMid = 3, kCfgMid2 = 4, kCfgBigS2 = 5, kCfgSmallS2 = 6, kCfgWhole = 7 };
+enum { kCfgBig = 0, kCfgTiny = 2, kCfgMid = 3, kCfgMid2 = 4, kCfgBigS2 = 5, kCfgSmallS2 = 6, kCfgWhole = 7, kCfgTiles = 8 };
 
 int64_t tiles_of(int64_t m, int64_t n, int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
 
@@ -747,6 +747,9 @@ hipError_t dispatch(const void *w, const void *a, float *c, const MfmaPlan &plan
     case kCfgBigS2: return launch_kq<KqBigS2<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgSmallS2: return launch_kq<KqSmallS2<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgWhole: return launch_q4_K_small(w, a, c, m, n, k, stream);
+    case kCfgTiles:
+        return launch_kquant_gemv(T == Kq::Q4K ? PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K : PFNG_WEIGHT_IQ2_XXS_ACTIVATION_Q8_K,
+                                  w, a, c, m, n, k, stream);
     default: return launch_kq<KqTiny<T>, false>(w, a, c, nullptr, m, n, k, stream);
     }
 }
@@ -754,7 +757,8 @@ hipError_t dispatch(const void *w, const void *a, float *c, const MfmaPlan &plan
 }  // namespace
 
 // Tile choice (measured on MI355X, 256 CUs, n = 4096 and the baseline
-// shapes): q4_K at k = 1024 or 1536 with half to one 32 x 96 tile per CU: the
+// shapes): the 16-row tiles of gemv_kquant.hip for the small m they win
+// (kquant_tiles_as_gemm); q4_K at k = 1024 or 1536 with half to one 32 x 96 tile per CU: the
 // whole-K tiles of gemm_small.hip (c2: 7.60 against 8.59 us for the 64 x 64
 // tiles with 2 slices); 128 x 64 tiles at two or more per CU; with 2
 // super-block slices at one or more per CU (c3); 64 x 64 tiles with 2 slices
@@ -762,8 +766,9 @@ hipError_t dispatch(const void *w, const void *a, float *c, const MfmaPlan &plan
 // whole-K tiles: 9.1 instead of 11.3 us); below that the 32 x 32 tile with the
 // most slices (4, 2, 1) that keeps the waves at or under 8 per CU (more slices
 // only added barrier and staging work). The block-sum diagnostic of the
-// whole-K plan reports the 64 x 64 two-slice tiles' sums (the whole-K tiles
-// split super-blocks between K slices and add the parts only in fp32).
+// whole-K and the 16-row plans reports the 64 x 64 two-slice tiles' sums (the
+// whole-K tiles split super-blocks between K slices and add the parts only in
+// fp32).
 MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus) {
     MfmaPlan p;
     const int64_t c = cus;
@@ -771,7 +776,9 @@ MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus) {
     const int64_t wk = q4k ? 2 : 1;  // KqTiny's K-waves
     const int64_t t32 = tiles_of(m, n, 32, 32), t64 = tiles_of(m, n, 64, 64), t128 = tiles_of(m, n, 128, 64);
     const int64_t t96 = tiles_of(m, n, 32, 96);
-    if (q4k && q4_K_small_supported(k) && 2 * t96 >= c && t96 <= c)
+    if (kquant_tiles_as_gemm(type, m, n, k, cus))
+        p.config = kCfgTiles;
+    else if (q4k && q4_K_small_supported(k) && 2 * t96 >= c && t96 <= c)
         p.config = kCfgWhole;
     else if (t128 >= 2 * c)
         p.config = kCfgBig;
@@ -809,6 +816,7 @@ hipError_t dispatch_isums(const void *w, const void *a, int32_t *out, const Mfma
     case kCfgBig: return launch_kq<KqIsums<KqBig<T>>, true>(w, a, nullptr, out, m, n, k, stream);
     case kCfgBigS2: return launch_kq<KqIsums<KqBigS2<T>>, true>(w, a, nullptr, out, m, n, k, stream);
     case kCfgSmallS2:
+    case kCfgTiles:
     case kCfgWhole: return launch_kq<KqIsums<KqSmallS2<T>>, true>(w, a, nullptr, out, m, n, k, stream);
     case kCfgMid: return launch_kq<KqIsums<KqMid<T>>, true>(w, a, nullptr, out, m, n, k, stream);
     case kCfgMid2: return launch_kq<KqIsums<KqMid2<T>>, true>(w, a, nullptr, out, m, n, k, stream);

@@ -25,6 +25,8 @@
 // parts (2 s_j + 1) * S_j are added across the lanes first, so the super-block
 // sum is complete and exact before it is scaled by 0.125 * d * ad (the bound
 // of this format is per super-block).
+#include <type_traits>
+
 #include "device_common.h"
 #include "kernels.h"
 #include "pfng_iq2xxs_grid.h"
@@ -1082,16 +1084,42 @@ __host__ __device__ constexpr int q4k_chunk_lds_bytes(int c) {
     return kKqMfWaves * kChunkWaveBytes + (c == 1 ? kChunkPartialBytes : 0);
 }
 
+// The 16 waves' partials, kStride floats apart, added in T in pairs (a fixed
+// order). Relative error from 64 bits on random layers against fp32 sums in wave
+// order (k = 4096) or the GEMM tiles' slices (k = 2816): q4_K 1.03e-7 -> 8.7e-8 and
+// 9.1e-8 -> 8.5e-8, iq2_xxs 8.4e-8 -> 6.5e-8 and 6.0e-8 -> 6.3e-8 in fp32; in fp64
+// 7.2e-8, 7.2e-8, 4.3e-8 and 4.3e-8, for 1-2 % of the time (4096 x 4096, m = 128
+// q4_K 15.35 -> 15.49 us). So the iq2_xxs rows that the GEMM slices used to add
+// take fp64, the others fp32, which costs nothing.
+template <int kStride, class T = float>
+__device__ __forceinline__ float sum_wave_partials(const float *p) {
+    T v[kKqMfWaves];
+#pragma unroll
+    for (int i = 0; i < kKqMfWaves; ++i) v[i] = (T)p[i * kStride];
+#pragma unroll
+    for (int step = 1; step < kKqMfWaves; step *= 2)
+#pragma unroll
+        for (int i = 0; i < kKqMfWaves; i += 2 * step) v[i] += v[i + step];
+    return (float)v[0];
+}
+
 template <int C, int kG>
 __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(const uint8_t *__restrict__ w,
                                                                              const uint8_t *__restrict__ a,
                                                                              float *__restrict__ c, int m, int n,
                                                                              int groups) {
     static_assert(C >= 1 && C <= kMaxGemvChunks, "at most kMaxGemvChunks chunks of 16 activation rows");
-    // super-blocks of a row (k == 256 nsb, nsb % 4 == 0): kG when it
-    // is fixed at compile time (k = 4096: one round, constant strides), else groups
+    // super-blocks of a row (k == 256 nsb): kG when it is fixed at compile time
+    // (k = 4096: one round, constant strides), else groups
     const int nsb = kG > 0 ? kG : groups;
     const uint32_t kARow = (uint32_t)nsb * kQ8KBytes;
+    // The q8_K blocks are copied from o bytes before them, H1 from byte h1s of
+    // that. With nsb % 4 == 0 a wave's blocks lie alike in every row and o takes
+    // the copies to 16-byte boundaries (H1 = chunks 8..18); otherwise they start
+    // at the block, on a dword, and H1 is the block's last 176 bytes (chunks
+    // 8..18 would end 12 past it, for the last block past the rows).
+    const bool even_rows = kG > 0 ? kG % 4 == 0 : nsb % 4 == 0;
+    const int h1s = even_rows ? 128 : 116;
     constexpr int kH = run_copies<16, 11>();  // instructions per half (H1: 11 columns, H0: 9)
     static_assert(run_copies<16, 9>() == kH && run_copies<16, 9>() * 1024 <= 3072, "3 KB per run");
     static_assert(4 * C * 64 * 4 <= kChunkWaveBytes, "a wave's partials fit its buffers");
@@ -1100,7 +1128,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int n0 = blockIdx.x * 16;
-    const int o = 4 * (wave & 3);
+    const int o = even_rows ? 4 * (wave & 3) : 0;
     uint8_t *wl = lds + wave * kChunkWaveBytes, *h0 = wl + 3072, *h1 = wl + 6144;
     float acc[C][4];
 #pragma unroll
@@ -1126,7 +1154,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
         const int sb = kKqMfWaves * rnd + wave;
         const uint8_t *asrc = a + sb * kQ8KBytes - o;  // copy start of the wave's block in activation row 0
         auto copy_h0 = [&](int ch) { copy_run<C, 16, 9>(asrc + (size_t)ch * 16 * kARow, kARow, 0, m - 16 * ch, h0, cl); };
-        auto copy_h1 = [&](int ch) { run_copy<16, 11>(asrc + (size_t)ch * 16 * kARow, kARow, 8, m - 16 * ch, h1, cl); };
+        auto copy_h1 = [&](int ch) { run_copy<16, 11>(asrc + (size_t)ch * 16 * kARow + h1s, kARow, 0, m - 16 * ch, h1, cl); };
         copy_run<C, 16, 9>(w + ((size_t)n0 * nsb + sb) * 144, nsb * 144, 0, n - n0, wl, cl);
         copy_h0(0);
         copy_h1(0);
@@ -1149,8 +1177,8 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
         const _Float16 m0 = (_Float16)(int)(mp & 0xffu), m1 = (_Float16)(int)((mp >> 8) & 0xffu);
         const f16x4 mm = {m0, m0, m1, m1};
         const float d = fp16_to_f32(hd.x & 0xffffu), dmin = fp16_to_f32(hd.x >> 16);
-        // activation byte b of chunk row r: H0 at h0 + 144 r + o + b, H1 at h1 + 176 r + o + b - 128
-        const uint8_t *a0 = h0 + li * 144 + o + 4 + 4 * q, *a1 = h1 + li * 176 + o - 128 + 4 + 4 * q;
+        // activation byte b of chunk row r: H0 at h0 + 144 r + o + b, H1 at h1 + 176 r + o + b - h1s
+        const uint8_t *a0 = h0 + li * 144 + o + 4 + 4 * q, *a1 = h1 + li * 176 + o - h1s + 4 + 4 * q;
     #pragma unroll
         for (int ch = 0; ch < C; ++ch) {
             if (ch > 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kH) : "memory");  // H0(ch)
@@ -1193,7 +1221,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
     }
     // wave partials through LDS, each wave's in a region only it writes
     // ([group g = 4 chunk + r][lane]); wave w adds groups w, w + 16, ... over
-    // the waves in wave order and stores them
+    // the waves and stores them
     const int li = lane & 15, q = lane >> 4;
     // wave v's partials at red + v * kStride: a compile-time stride, so the
     // reads below take immediate offsets from one address
@@ -1206,14 +1234,13 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
     __syncthreads();
     const int col = n0 + li;
     for (int g = wave; g < 4 * C; g += kKqMfWaves) {
-        float s = red[g * 64 + lane];
-        for (int v = 1; v < kKqMfWaves; ++v) s += red[v * kStride + g * 64 + lane];
+        const float s = sum_wave_partials<kStride>(red + g * 64 + lane);
         const int row = 16 * (g / 4) + 4 * q + g % 4;
         if (col < n && row < m) store_through(&c[(size_t)row * n + col], s);
     }
 }
 
-// iq2_xxs, from k = 4096 at k % 2048 == 0: as gemv_q4_K_mfma_chunk_kernel, with the
+// iq2_xxs: as gemv_q4_K_mfma_chunk_kernel, with the
 // weight decode of gemv_iq2_xxs_mfma_sb_kernel done once per wave (5 weight
 // columns per row, H1 = activation chunks 8..16). Every wave copies the grid
 // and sign tables into its own LDS region before everything else and reads
@@ -1229,14 +1256,17 @@ __host__ __device__ constexpr int iq2_chunk_lds_bytes(int c) {
     return kKqMfWaves * kIq2ChunkWaveBytes + (c == 1 ? kChunkPartialBytes : 0);
 }
 
-template <int C, int kG>
+template <int C, int kG, bool kAnyK = false>
 __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_iq2_xxs_mfma_chunk_kernel(const uint8_t *__restrict__ w,
                                                                                 const uint8_t *__restrict__ a,
                                                                                 float *__restrict__ c, int m, int n,
                                                                                 int groups) {
     static_assert(C >= 1 && C <= kMaxGemvChunks, "at most kMaxGemvChunks chunks of 16 activation rows");
-    // super-blocks of a row (k == 256 nsb, nsb % 8 == 0): kG when it
-    // is fixed at compile time (k = 4096: one round, constant strides), else groups
+    // super-blocks of a row (k == 256 nsb): kG when it is fixed at compile time
+    // (k = 4096: one round, constant strides), else groups. kAnyK false: nsb is
+    // a multiple of 8, and every row's blocks lie at the same offset from a
+    // 16-byte boundary (per-lane offsets instead: 11.45 against 11.21 us at
+    // m = 16, 4096 x 14336)
     const int nsb = kG > 0 ? kG : groups;
     const uint32_t kARow = (uint32_t)nsb * kQ8KBytes;
     constexpr int kH = run_copies<16, 9>();  // instructions per copy (run_copy_exact issues as many)
@@ -1247,7 +1277,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_iq2_xxs_mfma_chunk_kerne
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int n0 = blockIdx.x * 16;
-    const int o2 = 2 * (wave & 7), o = 4 * (wave & 3);
+    const int o = kAnyK ? 0 : 4 * (wave & 3);  // bytes from a copy's start to its q8_K block
     uint8_t *grid = lds + wave * kIq2ChunkWaveBytes;  // grid magnitudes, then sign masks
     uint8_t *wl = grid + kIq2TableBytes, *h0 = wl + kIq2ChunkRunW, *h1 = h0 + kIq2ChunkRunH;
     static_assert(kIq2TableBytes == 3 * 1024, "three 1-KB table pieces");
@@ -1286,7 +1316,24 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_iq2_xxs_mfma_chunk_kerne
         auto copy_h1 = [&](int ch) {
             run_copy_exact<16, 9>(asrc + (size_t)ch * 16 * kARow, kARow, 8, m - 16 * ch, h1, cl);
         };
-        run_copy_exact<16, 5>(w + ((size_t)n0 * nsb + sb) * kIq2Bytes - o2, nsb * kIq2Bytes, 0, n - n0, wl, cl);
+        // The weight blocks (66 bytes at any even address) are copied as 5 chunks
+        // from o2 bytes before them: at nsb % 8 == 0 from a 16-byte boundary, where
+        // o2 = 2 (v % 8) in every row; otherwise from a dword, 2 bytes back where
+        // the block's index is odd and 12 more behind a row's first block, so that
+        // the chunks end at most 2 bytes past the block and only where the index
+        // is even: inside the matrix when its block count is even or the block is
+        // not its last (kq_tiles_take).
+        int o2;
+        if constexpr (!kAnyK) {
+            o2 = 2 * (wave & 7);
+            run_copy_exact<16, 5>(w + ((size_t)n0 * nsb + sb) * kIq2Bytes - o2, nsb * kIq2Bytes, 0, n - n0, wl, cl);
+        } else {
+            const int back = sb > 0 ? 12 : 0;
+            run_copy_exact<16, 5, true>(w + ((size_t)n0 * nsb + sb) * kIq2Bytes - back - 2, nsb * kIq2Bytes, 0, n - n0,
+                                        wl, cl, nsb & 1, sb);  // n0 is even
+            const int row = li < n - n0 ? li : n - n0 - 1;
+            o2 = back + 2 * ((sb + row * nsb) & 1);
+        }
         copy_h0(0);
         copy_h1(0);
         // weights and H0(0) (and, issued before them, the table copies)
@@ -1344,7 +1391,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_iq2_xxs_mfma_chunk_kerne
     }
     // wave partials through LDS, each wave's in a region only it writes
     // ([group g = 4 chunk + r][lane]); wave w adds groups w, w + 16, ... over
-    // the waves in wave order and stores them
+    // the waves and stores them
     const int li = lane & 15, q = lane >> 4;
     // wave v's partials at red + v * kStride: a compile-time stride, so the
     // reads below take immediate offsets from one address
@@ -1361,8 +1408,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_iq2_xxs_mfma_chunk_kerne
     __syncthreads();
     const int col = n0 + li;
     for (int g = wave; g < 4 * C; g += kKqMfWaves) {
-        float s = red[g * 64 + lane];
-        for (int v = 1; v < kKqMfWaves; ++v) s += red[v * kStride + g * 64 + lane];
+        const float s = sum_wave_partials<kStride, std::conditional_t<kAnyK, double, float>>(red + g * 64 + lane);
         const int row = 16 * (g / 4) + 4 * q + g % 4;
         if (col < n && row < m) store_through(&c[(size_t)row * n + col], s);
     }
@@ -1382,18 +1428,29 @@ void launch_kq_chunk(bool q4k, const uint8_t *w, const uint8_t *a, float *c, int
     else if (nsb == kKqMfWaves)
         hipLaunchKernelGGL((gemv_iq2_xxs_mfma_chunk_kernel<C, kKqMfWaves>), grid, block, lds, stream, w, a, c, m, n,
                            nsb);
-    else
+    else if (nsb % 8 == 0)
         hipLaunchKernelGGL((gemv_iq2_xxs_mfma_chunk_kernel<C, 0>), grid, block, lds, stream, w, a, c, m, n, nsb);
+    else
+        hipLaunchKernelGGL((gemv_iq2_xxs_mfma_chunk_kernel<C, 0, true>), grid, block, lds, stream, w, a, c, m, n, nsb);
 }
 
-// k the chunked MFMA tile kernels take: every row's blocks at the same offset
-// from a 16-byte boundary, with the last block's copy ending at the row's end
-// (q4_K: k % 1024 == 0, the q8_K blocks' offset set by the block index mod 4;
-// iq2_xxs: k % 2048 == 0, its 66-byte weight blocks' offset by the index mod
-// 8). Below k = 4096 the waves past the last super-block idle.
+// k that the chunked MFMA tile kernels have always taken as GEMVs up to
+// gemv_tiles_max_m: every row's blocks at the same offset from a 16-byte
+// boundary (q4_K: k % 1024 == 0, the q8_K blocks' offset set by the block index
+// mod 4; iq2_xxs: k % 2048 == 0, its 66-byte weight blocks' offset by the index
+// mod 8). Below k = 4096 the waves past the last super-block idle.
 bool kq_tiles_take_k(int type, int64_t k) {
     const int64_t unit = type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K ? 1024 : 2048;
     return k % unit == 0 && k >= unit;
+}
+
+// Shapes those kernels can run: any k from 1024 (q4_K) or 2048 (iq2_xxs), the
+// latter with an even number of weight blocks (the copy of the last block may
+// read the dword its last two bytes lie in, which is then inside the matrix).
+// An odd count (n and k / 256 both odd) keeps the other kernels.
+bool kq_tiles_take(int type, int64_t n, int64_t k) {
+    if (type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K) return k % 256 == 0 && k >= 1024;
+    return k % 256 == 0 && k >= 2048 && n * (k / 256) % 2 == 0;
 }
 
 // Smallest m from which the one-chunk tile runs, measured at n = 4096 against
@@ -1404,7 +1461,9 @@ bool kq_tiles_take_k(int type, int64_t k) {
 // k = 4096 from m = 9, m = 5..8 taking the two-half-copy kernel (4096 x 4096
 // against the staged kernel, us: m = 4 5.23 / 5.08, m = 5 5.34 / 5.91, m = 8
 // 5.56 / 6.58); above 4096 m = 5 (k = 8192 m = 5 8.29 / 9.46, m = 12 8.87 /
-// 16.72; k = 14336 m = 8 12.54 / 18.98).
+// 16.72; k = 14336 m = 8 12.54 / 18.98). Other k alike: q4_K k = 1280 m = 8 3.19
+// / 5.17, k = 2560 m = 4 3.84 / 4.11, k = 11008 m = 5 7.41 / 9.87, m = 8 8.10 /
+// 13.28; iq2_xxs k = 2560 m = 5 4.10 / 5.23, k = 11008 m = 8 8.75 / 14.36.
 int kq_tiles_min_m(int type, int64_t k) {
     if (type == PFNG_WEIGHT_IQ2_XXS_ACTIVATION_Q8_K) return k == 4096 ? 9 : 5;
     if (k <= 1024) return 3;
@@ -1419,7 +1478,7 @@ hipError_t launch_kq_gemv(int type, const void *w, const void *a, float *c, int6
     const int64_t nsb = k / 256;
     if constexpr (M >= 3) {
         // one chunk of the chunked kernel from m = kq_tiles_min_m(type, k)
-        if (M >= kq_tiles_min_m(type, k) && kq_tiles_take_k(type, k)) {
+        if (M >= kq_tiles_min_m(type, k) && kq_tiles_take(type, n, k)) {
             launch_kq_chunk<1>(type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K, wp, ap, c, M, (int)n, (int)nsb, stream);
             return hipGetLastError();
         }
@@ -1507,6 +1566,20 @@ bool kquant_gemv_chunked_fits(int type, int64_t m, int64_t k) {
     return m >= 9 && m <= gemv_tiles_max_m(k) && kq_tiles_take_k(type, k);
 }
 
+// Against the GEMM tiles (us, tiles of 16 weight rows / GEMM): q4_K k = 11008,
+// n = 4096, m = 16 9.4 / 23.4, m = 37 15.2 / 25.4, m = 64 20.1 / 26.5, m = 100
+// 29.5 / 55.1, m = 128 35.4 / 56.9; iq2_xxs m = 16 9.5 / 29.0, m = 100 26.9 /
+// 59.3, m = 128 31.2 / 59.8. Their time goes with the rounds of 16-row tiles, one
+// per CU, so wide outputs from m = 17 stay with the GEMM: k = 2304, n = 11008 (3
+// rounds) m = 100 q4_K 23.6 / 29.5, iq2_xxs 22.8 / 26.2, but n = 14336 (4 rounds)
+// 30.9 / 29.8 and 29.9 / 26.4; k = 1280 q4_K n = 8192 (2 rounds) m = 64 9.8 /
+// 11.3, n = 11008 14.0 / 11.6.
+bool kquant_tiles_as_gemm(int type, int64_t m, int64_t n, int64_t k, int cus) {
+    if (m < kq_tiles_min_m(type, k) || m > gemv_tiles_max_m(k)) return false;
+    if (kq_tiles_take_k(type, k) || !kq_tiles_take(type, n, k)) return false;
+    return m <= 16 || (n + 15) / 16 <= (int64_t)cus * (k >= 2048 ? 3 : 2);
+}
+
 hipError_t launch_kquant_gemv(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                               hipStream_t stream) {
     if (type != PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K && type != PFNG_WEIGHT_IQ2_XXS_ACTIVATION_Q8_K)
@@ -1530,7 +1603,7 @@ hipError_t launch_kquant_gemv(int type, const void *w, const void *a, float *c, 
     case 16: return launch_kq_gemv<16>(type, w, a, c, n, k, stream);
     default: break;
     }
-    if (!kquant_gemv_chunked_fits(type, m, k)) return hipErrorInvalidValue;
+    if (m < 17 || m > gemv_tiles_max_m(k) || !kq_tiles_take(type, n, k)) return hipErrorInvalidValue;
     const auto *wp = static_cast<const uint8_t *>(w);
     const auto *ap = static_cast<const uint8_t *>(a);
     const bool q4k = type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K;

@@ -43,6 +43,9 @@ bool kquant_gemv_staged_fits(int64_t m, int64_t k);
 // m = 9..gemv_tiles_max_m(k) at q4_K k % 1024 == 0, iq2_xxs k % 2048 == 0: MFMA tiles of 16
 // weight rows over chunks of 16 activation rows
 bool kquant_gemv_chunked_fits(int type, int64_t m, int64_t k);
+// shapes outside those GEMV rules that the MFMA path runs on the same tiles:
+// the other k from 1024 (q4_K) or 2048 (iq2_xxs), up to the same m
+bool kquant_tiles_as_gemm(int type, int64_t m, int64_t n, int64_t k, int cus);
 hipError_t launch_kquant_gemv(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                               hipStream_t stream);
 
