@@ -44,7 +44,8 @@ typedef enum {
 /* Matrix-product implementations; PFNG_PATH_AUTO picks per shape (the GEMV
  * where it applies: up to m = 16, and its MFMA tiles up to m = 64 below
  * k = 2048 and m = 128 from there, for q4_0 at k % 256 == 0 from 512, q4_K at
- * k % 1024 == 0, iq2_xxs at k % 2048 == 0; then the MFMA GEMM tiles) and
+ * k % 1024 == 0, iq2_xxs at k % 2048 == 0, except where n is so wide, from m = 17
+ * and n > 4096, that the GEMM is predicted faster; then the MFMA GEMM tiles) and
  * returns PFNG_ERR_UNSUPPORTED when neither applies (see pfng_hip_auto_path). */
 typedef enum {
     PFNG_PATH_AUTO = 0,

@@ -206,12 +206,14 @@ int pfng_hip_mul_mat(int type, const void *weight, const void *act_q, float *out
     switch (path) {
     case PFNG_PATH_AUTO:
         // measured at 4096x4096: every GEMV that applies (up to m = 128 at the
-        // tiles' k) is faster than the MFMA GEMM. When neither tiled path takes the shape
+        // tiles' k) is faster than the MFMA GEMM; on wider outputs the predicted
+        // times decide (mfma_preferred). When neither tiled path takes the shape
         // the call is declined (as the reference's validate_shape declines,
         // kernels/common/adapter_common.h:28-43) instead of dropping to the
         // one-thread-per-output kernel, which is 10-500x slower; the caller
         // may ask for PFNG_PATH_NAIVE explicitly.
-        if (gemv_ok) return hip_status(pfng::launch_gemv(type, weight, act_q, out, m, n, k, s), "gemv launch");
+        if (gemv_ok && !(mfma_ok && pfng::mfma_preferred(type, m, n, k)))
+            return hip_status(pfng::launch_gemv(type, weight, act_q, out, m, n, k, s), "gemv launch");
         if (mfma_ok) return launch_mfma(type, weight, act_q, out, m, n, k, s);
         if (!base_aligned)
             return fail(PFNG_ERR_UNSUPPORTED,
@@ -246,8 +248,9 @@ int pfng_hip_mul_mat(int type, const void *weight, const void *act_q, float *out
 int pfng_hip_auto_path(int type, int64_t m, int64_t n, int64_t k) {
     if (check_shape(type, m, n, k)) return -1;
     if (m == 0 || n == 0) return PFNG_PATH_AUTO;
-    if (pfng::gemv_supported(type, m, k)) return PFNG_PATH_GEMV;
-    if (pfng::mfma_supported(type, m, k)) return PFNG_PATH_MFMA;
+    const bool mfma_ok = pfng::mfma_supported(type, m, k);
+    if (pfng::gemv_supported(type, m, k) && !(mfma_ok && pfng::mfma_preferred(type, m, n, k))) return PFNG_PATH_GEMV;
+    if (mfma_ok) return PFNG_PATH_MFMA;
     fail(PFNG_ERR_UNSUPPORTED,
          "%s: no tiled path takes m=%lld k=%lld (%s; %s; both k <= %lld); PFNG_PATH_NAIVE runs every shape in "
          "the reference's fp32 order",

@@ -28,11 +28,13 @@
 // 200x4096x11008 51.6 -> 48.7. Loading the pieces from their own byte address
 // (two past a dword for every other block), which needs no realignment, is
 // slower (269.5 against 261.0 and 35.9 against 29.0 us).
-// Small problems use 32x32 tiles whose stage blocks are shared by two waves
-// (their partial sums are added through LDS at the end), so that even a few
-// hundred output tiles keep several waves resident on every CU.
+// Smaller problems use smaller tiles whose stage blocks are shared by several
+// K-waves (their partial sums are added through LDS at the end), so that one
+// workgroup keeps eight waves on its CU.
 //
 // A diagnostic instantiation writes S_b instead of accumulating (block isums).
+#include <type_traits>
+
 #include "device_common.h"
 #include "kernels.h"
 
@@ -48,12 +50,18 @@ constexpr uint32_t kBufferWord3 = 0x00020000;  // raw buffer resource
 // AHEAD staging pieces per thread are in flight (a stage has kPieces of them:
 // a deep prefetch for the small tiles, whose stages are too short to cover a
 // memory round trip).
-template <int BM, int BN, int WM, int WN, int KB, int WK = 1, int AHEAD = 6, int MINW = 2>
+// FOLD: the accumulators are added into a second set after every two stages, so
+// that no fp32 sum runs over more than a few dozen terms (these tiles take over
+// shapes of the 16-wave tile GEMV, whose sums are that short). It costs no time;
+// relative error from 64 bits on random layers: 100x11008x4096 1.47e-7 without,
+// 9.3e-8 with (9.4e-8 in the tile GEMV), 333x4096x4096 2.0e-7 -> 9.3e-8.
+template <int BM, int BN, int WM, int WN, int KB, int WK = 1, int AHEAD = 6, bool FOLD = false, int MINW = 2>
 struct Q40Config {
     static constexpr int kBM = BM, kBN = BN, kWM = WM, kWN = WN, kKB = KB, kWK = WK, kAhead = AHEAD;
     // waves per SIMD the register budget must allow: the fp32 epilogue needs two
     // resident waves per SIMD to keep the VALU issuing while the other waits
     static constexpr int kMinWavesPerEU = MINW;
+    static constexpr bool kFold = FOLD;
     static constexpr int kThreads = 64 * WM * WN * WK;
     static constexpr int kWaveBlocks = KB / WK;  // blocks per stage of one wave
     static constexpr int TM = BM / WM / 32;  // 32x32 tiles per wave along m
@@ -108,8 +116,14 @@ struct PieceRegs {
 // values sit two bytes off. Either way the piece is bytes [2, 18) or [4, 20) of
 // the five dwords from the one at or before its block (half), none of which
 // lies past the block pair's end.
+// Where nb is not a multiple of KB, the last stage's loads of blocks past the
+// row's end are sent out of the resource (to kPastEnd: the largest, 128 rows of
+// 2^24 elements, ends below it) and read zeros: a zero scale on both sides, so
+// such a block adds S * 0.
+constexpr uint32_t kPastEnd = 0xf0000000u;
 struct StageSlots {
     uint32_t a, w;               // load offsets of piece 0
+    uint32_t a_last, w_last;     // the same in the last stage: kPastEnd where its block lies past the row
     uint32_t sel_a, sel_w;       // v_perm selectors: bytes [2, 6) or [4, 8) of a dword pair
     uint32_t ad_shift, wd_mask;  // the scale's place in dword 0
     int aq, ad, ad_step, wq, wd; // LDS places of piece 0, within a stage buffer
@@ -124,6 +138,9 @@ __device__ __forceinline__ StageSlots stage_slots(int nb) {
     o.a = (uint32_t)ra * (uint32_t)nb * 34u + ((34u * (uint32_t)ja + 16u * (uint32_t)ha) & ~3u);
     const int rw = threadIdx.x / C::kWPerRow, jw = threadIdx.x % C::kWPerRow;
     o.w = (uint32_t)rw * (uint32_t)nb * 18u + ((18u * (uint32_t)jw) & ~3u);
+    const int tail = nb % C::kKB;
+    o.a_last = tail && ja >= tail ? kPastEnd : o.a;
+    o.w_last = tail && jw >= tail ? kPastEnd : o.w;
     o.sel_a = ja & 1 ? kOdd : kEven;
     o.sel_w = jw & 1 ? kOdd : kEven;
     o.ad_shift = ja & 1 ? 16 : 0;
@@ -145,14 +162,15 @@ __device__ __forceinline__ void load5(__amdgpu_buffer_rsrc_t r, uint32_t voffset
 }
 
 // Load / store of piece p (activation pieces first). kb: the stage's first
-// block; buf: the stage's LDS buffer.
+// block; last: whether it is the last stage; buf: the stage's LDS buffer.
 template <class C>
 __device__ __forceinline__ void load_piece(__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rw, const StageSlots &o,
-                                           int nb, int kb, int p, PieceRegs &r) {
+                                           int nb, int kb, bool last, int p, PieceRegs &r) {
     if (p < C::kActPT)
-        load5(ra, o.a, (uint32_t)(p * C::kActRows) * (uint32_t)nb * 34u + (uint32_t)kb * 34u, r.v);
+        load5(ra, last ? o.a_last : o.a, (uint32_t)(p * C::kActRows) * (uint32_t)nb * 34u + (uint32_t)kb * 34u, r.v);
     else
-        load5(rw, o.w, (uint32_t)((p - C::kActPT) * C::kWRows) * (uint32_t)nb * 18u + (uint32_t)kb * 18u, r.v);
+        load5(rw, last ? o.w_last : o.w,
+              (uint32_t)((p - C::kActPT) * C::kWRows) * (uint32_t)nb * 18u + (uint32_t)kb * 18u, r.v);
 }
 
 template <class C>
@@ -238,7 +256,8 @@ struct ItemRegs {
 // even distances along the list, behind the MFMAs of the next item: the next
 // stage's pieces go to the other LDS buffer and the loads after them go out
 // while the matrix cores work, instead of in a phase of their own.
-template <class C, bool kIsums, class Piece>
+// fresh: the accumulators start over with the stage's first block.
+template <class C, bool kIsums, bool kFresh, class Piece>
 __device__ __forceinline__ void compute_stage(uint8_t *lds, int buf, f32x16 (&acc)[C::TM][C::TN], int32_t *isums,
                                               int m, int n, int nb, int m0, int n0, int s, int tb, int lane,
                                               int wave_m, int wave_n, Piece piece) {
@@ -308,11 +327,14 @@ __device__ __forceinline__ void compute_stage(uint8_t *lds, int buf, f32x16 (&ac
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
                 const int row = m0 + wave_m * C::TM * 32 + tm * 32 + mfma_row(lane, q);
-                if (row < m && col < n) isums[((size_t)row * n + col) * nb + s * C::kKB + tb + t] = r.s16[q] / 16;
+                const int blk = s * C::kKB + tb + t;
+                if (row < m && col < n && blk < nb) isums[((size_t)row * n + col) * nb + blk] = r.s16[q] / 16;
             }
         } else {
 #pragma unroll
-            for (int q = 0; q < 16; ++q) acc[tm][tn][q] = fmaf(based_sum(r.s16[q]), r.p[q], acc[tm][tn][q]);
+            for (int q = 0; q < 16; ++q)
+                acc[tm][tn][q] = kFresh && t == 0 ? based_sum(r.s16[q]) * r.p[q]
+                                                  : fmaf(based_sum(r.s16[q]), r.p[q], acc[tm][tn][q]);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -346,6 +368,23 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
     for (int i = 0; i < C::TM; ++i)
 #pragma unroll
         for (int j = 0; j < C::TN; ++j) acc[i][j] = (f32x16){};
+    f32x16 total[C::TM][C::TN];  // kFold
+    auto fold = [&]() __attribute__((always_inline)) {
+        if constexpr (C::kFold && !kIsums) {
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) total[i][j][q] += acc[i][j][q];
+        }
+    };
+    if constexpr (C::kFold && !kIsums) {
+#pragma unroll
+        for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < C::TN; ++j) total[i][j] = (f32x16){};
+    }
 
     // Double-buffered LDS with one barrier per stage: while stage s is computed
     // from one buffer, the pieces of stage s+1 go from registers into the
@@ -355,7 +394,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
     // divergent control flow; rounds of two stages make register set and
     // buffer compile-time constants, and an odd last stage is computed after
     // the loop.
-    const int stages = nb / C::kKB;
+    const int stages = (nb + C::kKB - 1) / C::kKB;
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(a + (size_t)m0 * nb * 34), 0,
         (int)((uint32_t)(m - m0 < C::kBM ? m - m0 : C::kBM) * (uint32_t)nb * 34u), kBufferWord3);
@@ -368,37 +407,53 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
     PieceRegs regs[C::kAhead];
     // piece x of the sequence over all stages
     auto load = [&](int st, int p, PieceRegs &r) __attribute__((always_inline)) {
-        load_piece<C>(ra, rw, slots, nb, (st < stages ? st : stages - 1) * C::kKB, p, r);
+        const int last = stages - 1;
+        load_piece<C>(ra, rw, slots, nb, (st < last ? st : last) * C::kKB, st >= last, p, r);
     };
     {
         PieceRegs first[C::kPieces];
 #pragma unroll
         for (int p = 0; p < C::kPieces; ++p) load(0, p, first[p]);
 #pragma unroll
+        for (int x = 0; x < C::kAhead; ++x) load(1 + x / C::kPieces, x % C::kPieces, regs[x]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
         for (int p = 0; p < C::kPieces; ++p) store_piece<C>(lds, slots, p, first[p]);
     }
-#pragma unroll
-    for (int x = 0; x < C::kAhead; ++x) load(1 + x / C::kPieces, x % C::kPieces, regs[x]);
     __syncthreads();
     const int tb = wk * C::kWaveBlocks;
     int s = 0;
+    // one stage of a round (R = 0 or 1), from buffer R
+    auto stage = [&](auto R) __attribute__((always_inline)) {
+        constexpr int rr = decltype(R)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        compute_stage<C, kIsums, C::kFold && rr == 0>(
+            lds, rr, acc, isums, m, n, nb, m0, n0, s + rr, tb, lane, wave_m, wave_n,
+            [&](int p) __attribute__((always_inline)) {
+                PieceRegs &r = regs[(rr * C::kPieces + p) % C::kAhead];
+                store_piece<C>(lds + (rr ^ 1) * C::kBufBytes, slots, p, r);
+                const int x = p + C::kAhead;
+                load(s + rr + 1 + x / C::kPieces, x % C::kPieces, r);
+            });
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
     for (; s + 1 < stages; s += 2) {
-#pragma unroll
-        for (int rr = 0; rr < 2; ++rr) {
-            __builtin_amdgcn_sched_barrier(0);
-            compute_stage<C, kIsums>(lds, rr, acc, isums, m, n, nb, m0, n0, s + rr, tb, lane, wave_m, wave_n,
-                                     [&](int p) __attribute__((always_inline)) {
-                                         PieceRegs &r = regs[(rr * C::kPieces + p) % C::kAhead];
-                                         store_piece<C>(lds + (rr ^ 1) * C::kBufBytes, slots, p, r);
-                                         const int x = p + C::kAhead;
-                                         load(s + rr + 1 + x / C::kPieces, x % C::kPieces, r);
-                                     });
-            __builtin_amdgcn_sched_barrier(0);
-            __syncthreads();
-        }
+        stage(std::integral_constant<int, 0>{});
+        stage(std::integral_constant<int, 1>{});
+        fold();
     }
-    if (s < stages)
-        compute_stage<C, kIsums>(lds, 0, acc, isums, m, n, nb, m0, n0, s, tb, lane, wave_m, wave_n, [](int) {});
+    if (s < stages) {
+        compute_stage<C, kIsums, C::kFold>(lds, 0, acc, isums, m, n, nb, m0, n0, s, tb, lane, wave_m, wave_n,
+                                           [](int) {});
+        fold();
+    }
+    if constexpr (C::kFold && !kIsums) {
+#pragma unroll
+        for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < C::TN; ++j) acc[i][j] = total[i][j];
+    }
 
     if constexpr (!kIsums) {
         if constexpr (C::kWK > 1) {
@@ -455,67 +510,135 @@ hipError_t launch_q4_0(const void *w, const void *a, float *c, int32_t *isums, i
     return hipGetLastError();
 }
 
-// large problems: 128x128 tiles, 4 waves of 64x64, 4 blocks per stage; half a
+// The tiles, from large to small problems; every one takes any k % 128 == 0 (a
+// last stage that the row does not fill reads zeros).
+// 128x128, 4 waves of 64x64, 4 blocks per stage, two workgroups per CU; half a
 // stage's pieces in flight (all six would spill: the accumulators, two items'
 // results and the fragments leave no room)
 using Q40Big = Q40Config<128, 128, 2, 2, 4, 1, 3>;
-// medium problems: 64x64 tiles, 4 waves of 32x32, 8 blocks per stage
+// 128x64, 8 waves of 32x32, 8 blocks per stage (as 4 waves of 64x32 in 2 K-waves
+// it is no faster, and has no registers left to fold into)
+using Q40Mid = Q40Config<128, 64, 4, 2, 8, 1, 5, true>;
+// 64x64, 4 waves of 32x32 in 2 K-waves each taking 8 of a 16-block stage
+using Q40SmallK2 = Q40Config<64, 64, 2, 2, 16, 2, 6, true>;
+// 32x64, 2 waves of 32x32 in 4 K-waves each taking 4 of a 16-block stage
+using Q40WideK4 = Q40Config<32, 64, 1, 2, 16, 4, 8, true>;
+// 64x64, 4 waves of 32x32, 8 blocks per stage, two workgroups per CU (short k)
 using Q40Small = Q40Config<64, 64, 2, 2, 8>;
-// medium problems with k % 256 != 0: 64x64 tiles, 2 waves of 64x32, 4 blocks per stage
+// 64x64, 2 waves of 64x32, 4 blocks per stage, four workgroups per CU
 using Q40Small4 = Q40Config<64, 64, 1, 2, 4>;
-// small problems: 32x32 tiles, 2 waves each taking 4 of the stage's 8 blocks,
-// two stages' pieces in flight
-using Q40Tiny = Q40Config<32, 32, 1, 1, 8, 2, 12>;
+// 32x32, 2 K-waves each taking 4 of an 8-block stage, several workgroups per CU
+// (short k)
+using Q40Tiny = Q40Config<32, 32, 1, 1, 8, 2, 6>;
+// 32x32, one wave in 8 K-waves each taking 4 of a 32-block stage, two stages'
+// pieces in flight
+using Q40TinyK8 = Q40Config<32, 32, 1, 1, 32, 8, 12, true>;
 
-// decode batches (at most one 32x32 tile per CU): 32x32 tiles, 8 waves each
-// taking 4 of the stage's 32 blocks, two stages' pieces in flight
-using Q40Mid = Q40Config<32, 32, 1, 1, 32, 8, 12>;
-
-// between the two: 64x64 tiles, 4 waves of 32x32 twice over (2 K-waves each
-// taking 8 of a 16-block stage)
-using Q40SmallK2 = Q40Config<64, 64, 2, 2, 16, 2, 6>;
-
-enum { kCfgBig = 0, kCfgSmall = 1, kCfgSmall4 = 2, kCfgTiny = 3, kCfgMid = 4, kCfgSmallK2 = 5, kCfgWhole = 6 };
+enum {
+    kCfgBig = 0,
+    kCfgMid = 1,
+    kCfgSmallK2 = 2,
+    kCfgWideK4 = 3,
+    kCfgTinyK8 = 4,
+    kCfgSmall = 5,
+    kCfgTiny = 6,
+    kCfgSmall4 = 7,
+    kCfgTiles = 8,  // the first that is no tile of this file
+    kCfgWhole = 8
+};
 
 int64_t tiles_of(int64_t m, int64_t n, int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
+
+// Tile choice: the least predicted time. A workgroup of the K-split tiles has a
+// CU to itself, so they take rounds of one tile per CU; the 128x128 and the plain
+// 64x64 tile run two, the 2-wave tiles four workgroups per CU. Nanoseconds per
+// round beyond the launch, fixed and per element of k (padded to whole stages),
+// fitted to 47 shapes with each tile forced (m 32..2048, n 100..14336, k 128..11008;
+// mostly within 8 %), us there: k = 4096, one tile per CU 32x32 11, 32x64 12.7,
+// 64x64 17.5, 128x64 27.5, 128x128 60, two 88, four of the 2-wave 64x64 55; two
+// rounds 64x64 33.6, 128x64 53.6. Against the tile counts that chose before, among
+// the plain 64x64, the 2-K-wave 32x32 and 64x64, and the 128x128 tiles:
+// 333x4096x4096 30.7 -> 27.9 us, 128x4096x4096 19.9 -> 13.5, 100x11008x4096 30.8 ->
+// 27.6, 333x1536x4096 20.0 -> 16.7, 200x4096x11008 51.8 -> 39.5, 480x4096x11008
+// 80.3 -> 68.8, 130x8000x1664 22.2 -> 15.7, 480x4096x1536 14.0 -> 13.4.
+int64_t q4_0_tile_ns(int config, int64_t m, int64_t n, int64_t k, int cus) {
+    auto rounds = [&](int64_t bm, int64_t bn) { return (tiles_of(m, n, bm, bn) + cus - 1) / cus; };
+    auto padded = [&](int64_t unit) { return (k + unit - 1) / unit * unit; };
+    switch (config) {
+    case kCfgBig: {
+        const int64_t r = rounds(128, 128);
+        return r / 2 * (5000 + 198 * k / 10) + r % 2 * (3400 + 135 * k / 10);
+    }
+    case kCfgMid: return rounds(128, 64) * (2900 + 575 * padded(256) / 100);
+    case kCfgSmallK2: return rounds(64, 64) * (1700 + 335 * padded(512) / 100);
+    case kCfgSmall: {
+        const int64_t r = rounds(64, 64), p = padded(256);
+        return r / 2 * (1600 + 665 * p / 100) + r % 2 * (2200 + 465 * p / 100) * (r > 1 ? 4 : 5) / 5;
+    }
+    case kCfgSmall4: {
+        const int64_t r = rounds(64, 64), rest = r % 4;
+        return r / 4 * (2200 + 125 * k / 10) + (rest ? 1800 + (rest > 1 ? 105 : 83) * k / 10 : 0);
+    }
+    case kCfgWideK4: return rounds(32, 64) * (1800 + 22 * padded(512) / 10);
+    case kCfgTiny: {
+        const int64_t r = rounds(32, 32), p = padded(256), rest = r % 4;
+        return r / 4 * (1700 + 475 * p / 100) + (rest ? 800 + 310 * p / 100 + (rest - 1) * (300 + 55 * p / 100) : 0);
+    }
+    default: return rounds(32, 32) * (1900 + 175 * padded(1024) / 100);
+    }
+}
+
+// The q4_0 tile with the least predicted time (a later one, mostly smaller,
+// only if it is 3 % less).
+int64_t best_q4_0_tile(int64_t m, int64_t n, int64_t k, int cus, int &config) {
+    int64_t best = 0;
+    for (int c = kCfgBig; c < kCfgTiles; ++c) {
+        const int64_t ns = q4_0_tile_ns(c, m, n, k, cus);
+        if (c == kCfgBig || ns + ns * 3 / 100 < best) {
+            best = ns;
+            config = c;
+        }
+    }
+    return best;
+}
 
 }  // namespace
 
 bool mfma_supported(int type, int64_t m, int64_t k) {
     (void)m;
     if (k > kMaxTiledK) return false;  // 32-bit load offsets
-    if (type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0) return k % (32 * 4) == 0;  // Q40Small4 takes any k % 128 == 0
+    if (type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0) return k % (32 * 4) == 0;  // whole dwords per block pair, stages of 4 blocks
     // the super-block formats take any k % 256 == 0 (gemm_kquant.hip)
     return (type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K || type == PFNG_WEIGHT_IQ2_XXS_ACTIVATION_Q8_K) && k % 256 == 0;
 }
 
-// Tile choice (measured on MI355X, 256 CUs): when the 32x32 tiles number at
-// most one per CU (decode batches: m <= 64 at n = 4096), the 8-K-wave 32x32
-// tile; else 128x128 tiles when there are at least two per CU, 64x64 tiles
-// from 1.25 per CU, the 2-K-wave 64x64 tile from 0.75 per CU when K is long
-// enough for its 16-block stages (256x4096x4096: 22.6 instead of 26.8 us), and
-// the 2-K-wave 32x32 tile below that.
+// The tile GEMV (16 weight rows a workgroup, one workgroup per CU) repeats its
+// activation chunks in every round, so on wide outputs the GEMM tiles overtake
+// it from m = 17. Its time, by rounds of 16-row tiles and chunks C = m / 16: 1.7
+// us + rounds (2.0 + 1.5 C) (0.25 + 0.75 k / 4096) us. At k = 4096, us GEMV / GEMM:
+// n = 11008 m = 16 12.0 / 12.8, m = 37 20.4 / 17.2, m = 64 24.2 / 17.7, m = 100 36.3 /
+// 27.6; n = 14336 m = 37 29.1 / 17.7, m = 64 33.7 / 18.4, m = 100 49.2 / 28.9. A single
+// round (n <= 4096) keeps the GEMV: m = 64 9.9 / 11.1, m = 100 13.7 / 13.5.
+bool mfma_preferred(int type, int64_t m, int64_t n, int64_t k) {
+    if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 || m <= 16) return false;
+    const int64_t rounds = (n + 16 * kMi355xCus - 1) / (16 * kMi355xCus);
+    if (rounds < 2) return false;
+    const int64_t chunks = (m + 15) / 16;
+    const int64_t gemv = 1700 + rounds * (2000 + 1500 * chunks) * (1024 + 3 * k / 4) / 4096;
+    int config;
+    return 2000 + best_q4_0_tile(m, n, k, kMi355xCus, config) < gemv;
+}
+
 MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus) {
     if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0) return plan_kquant(type, m, n, k, cus);
     MfmaPlan p;
-    const int64_t enough = 2 * (int64_t)cus;
-    if (k % (32 * Q40Mid::kKB) == 0 && tiles_of(m, n, 32, 32) <= cus) {
-        p.config = kCfgMid;
-    } else if (q4_0_small_supported(k) && 2 * tiles_of(m, n, 32, 96) >= cus && tiles_of(m, n, 32, 96) <= cus) {
+    if (q4_0_small_supported(k) && 2 * tiles_of(m, n, 32, 96) >= cus && tiles_of(m, n, 32, 96) <= cus) {
         // whole-K 32x96 tiles, one per CU and one round (480x1536x1536:
-        // 8.6 us against 9.8 us for the 2-K-wave 32x32 tile)
+        // 7.0 us against 8.9 us for the 64x64 tile)
         p.config = kCfgWhole;
-    } else if (tiles_of(m, n, 128, 128) >= enough) {
-        p.config = kCfgBig;
-    } else if (k % (32 * Q40Small::kKB) != 0) {
-        p.config = kCfgSmall4;
-    } else if (4 * tiles_of(m, n, 64, 64) >= 5 * (int64_t)cus) {
-        p.config = kCfgSmall;
-    } else if (k % (32 * Q40SmallK2::kKB) == 0 && k >= 2048 && 4 * tiles_of(m, n, 64, 64) >= 3 * (int64_t)cus) {
-        p.config = kCfgSmallK2;
-    } else {
-        p.config = kCfgTiny;
+        return p;
     }
+    best_q4_0_tile(m, n, k, cus, p.config);
     return p;
 }
 
@@ -524,12 +647,14 @@ hipError_t launch_mfma_mul_mat(int type, const void *w, const void *a, float *c,
     if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0) return launch_kquant_mul_mat(type, w, a, c, m, n, k, plan, stream);
     switch (plan.config) {
     case kCfgBig: return launch_q4_0<Q40Big, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgSmall: return launch_q4_0<Q40Small, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgTiny: return launch_q4_0<Q40Tiny, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgMid: return launch_q4_0<Q40Mid, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgSmallK2: return launch_q4_0<Q40SmallK2, false>(w, a, c, nullptr, m, n, k, stream);
+    case kCfgWideK4: return launch_q4_0<Q40WideK4, false>(w, a, c, nullptr, m, n, k, stream);
+    case kCfgSmall: return launch_q4_0<Q40Small, false>(w, a, c, nullptr, m, n, k, stream);
+    case kCfgTiny: return launch_q4_0<Q40Tiny, false>(w, a, c, nullptr, m, n, k, stream);
+    case kCfgSmall4: return launch_q4_0<Q40Small4, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgWhole: return launch_q4_0_small(w, a, c, nullptr, m, n, k, stream);
-    default: return launch_q4_0<Q40Small4, false>(w, a, c, nullptr, m, n, k, stream);
+    default: return launch_q4_0<Q40TinyK8, false>(w, a, c, nullptr, m, n, k, stream);
     }
 }
 
@@ -539,12 +664,14 @@ hipError_t launch_mfma_block_isums(int type, const void *w, const void *a, int32
         return launch_kquant_block_isums(type, w, a, out, m, n, k, plan, stream);
     switch (plan.config) {
     case kCfgBig: return launch_q4_0<Q40Big, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgSmall: return launch_q4_0<Q40Small, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgTiny: return launch_q4_0<Q40Tiny, true>(w, a, nullptr, out, m, n, k, stream);
     case kCfgMid: return launch_q4_0<Q40Mid, true>(w, a, nullptr, out, m, n, k, stream);
     case kCfgSmallK2: return launch_q4_0<Q40SmallK2, true>(w, a, nullptr, out, m, n, k, stream);
+    case kCfgWideK4: return launch_q4_0<Q40WideK4, true>(w, a, nullptr, out, m, n, k, stream);
+    case kCfgSmall: return launch_q4_0<Q40Small, true>(w, a, nullptr, out, m, n, k, stream);
+    case kCfgTiny: return launch_q4_0<Q40Tiny, true>(w, a, nullptr, out, m, n, k, stream);
+    case kCfgSmall4: return launch_q4_0<Q40Small4, true>(w, a, nullptr, out, m, n, k, stream);
     case kCfgWhole: return launch_q4_0_small(w, a, nullptr, out, m, n, k, stream);
-    default: return launch_q4_0<Q40Small4, true>(w, a, nullptr, out, m, n, k, stream);
+    default: return launch_q4_0<Q40TinyK8, true>(w, a, nullptr, out, m, n, k, stream);
     }
 }
 

@@ -49,6 +49,9 @@ bool kquant_tiles_as_gemm(int type, int64_t m, int64_t n, int64_t k, int cus);
 hipError_t launch_kquant_gemv(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                               hipStream_t stream);
 
+// compute units of the MI355X, for the choice between paths (made without a device)
+constexpr int kMi355xCus = 256;
+
 // Launch plan of the MFMA GEMMs: the tile configuration for the shape.
 struct MfmaPlan {
     int config = 0;
@@ -56,6 +59,8 @@ struct MfmaPlan {
 
 // gemm_mfma.hip
 bool mfma_supported(int type, int64_t m, int64_t k);
+// of a shape both tiled paths take: whether the automatic path runs the GEMM
+bool mfma_preferred(int type, int64_t m, int64_t n, int64_t k);
 MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus);
 hipError_t launch_mfma_mul_mat(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                                const MfmaPlan &plan, hipStream_t stream);

@@ -1,9 +1,9 @@
 """q4_0 GEMM tiles: the staging pieces at their edges, bit for bit.
 
 Each tile configuration of csrc/gemm_mfma.hip at one, two, three and more K
-stages (an odd last stage is computed outside the loop, and prefetched pieces
-past the last stage are clamped to it) and with ragged m and n (rows past the
-edge read zeros). On the inputs of tests/exact_inputs.py every fp32 step is
+stages (an odd last stage is computed outside the loop, prefetched pieces past
+the last stage are clamped to it, and blocks past a row's end read zeros) and
+with ragged m and n (rows past the edge read zeros). On the inputs of tests/exact_inputs.py every fp32 step is
 exact, so the tolerance is zero."""
 from __future__ import annotations
 
@@ -15,13 +15,11 @@ from test_gpu_exact import assert_bits_equal, dev, say
 
 pytestmark = pytest.mark.gpu
 
-# (m, n, k): 128x128 tiles (from 512 of them), 64x64 tiles with 8-block
-# stages and with 4-block stages, with two K waves, 32x32 tiles
-CASES = [(2048, 4096, 128), (2000, 4100, 256), (1921, 4097, 384), (2048, 4096, 640),
-         (1000, 1500, 256), (961, 1473, 768), (1000, 1500, 1280),
-         (700, 1100, 128), (65, 33, 384), (250, 129, 640),
-         (200, 4100, 2560), (129, 4033, 2048),
-         (65, 70, 256), (33, 31, 768), (130, 300, 1280), (17, 33, 1024), (31, 95, 3072)]
+# one, two, three and more stages of the 128x128 tiles; then a grid over which
+# the plan picks every tile, at k that fill the last stage of some and not of others
+CASES = ([(2048, 4096, 128), (2000, 4100, 256), (1921, 4097, 384), (2048, 4096, 640)]
+         + [(m, n, k) for m in (9, 33, 100, 200, 333, 700) for n in (100, 1500, 4100) for k in (128, 384, 1152, 2176)]
+         + [(40, 4100, 4096), (130, 4033, 4224), (500, 4000, 1664), (1000, 1500, 1280)])
 
 
 @pytest.mark.parametrize("m,n,k", CASES, ids=[f"{m}x{n}x{k}" for m, n, k in CASES])
@@ -34,3 +32,15 @@ def test_staging_bit_exact(hip, torch_gpu, oracle, m, n, k):
     rows = np.unique(np.r_[0, m - 1, np.random.default_rng(m).choice(m, min(m, 24), replace=False)])
     expect = oracle.matmul(0, w, np.ascontiguousarray(aq[rows]), len(rows), n, k)
     assert_bits_equal(got.cpu().numpy()[rows], expect, f"{m}x{n}x{k} (|a| <= {r})")
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 70, 640), (200, 1000, 896), (100, 300, 2176), (250, 4000, 384), (9, 40, 1152)])
+def test_block_isums_partial_stage(hip, torch_gpu, oracle, m, n, k):
+    """Block sums where the last stage is partly past the row's end."""
+    torch = torch_gpu
+    say(f"block isums q4_0 {m}x{n}x{k}")
+    act, w = oracle.create_input(0, m, n, k, seed=5)
+    aq = oracle.quantize_q8_0(act)
+    got = hip.block_isums(0, dev(torch, w), dev(torch, aq), m, n, k)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), oracle.isums(0, w, aq, m, n, k))
