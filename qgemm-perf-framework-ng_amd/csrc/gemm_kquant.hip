@@ -710,17 +710,13 @@ hipError_t launch_kq(const void *w, const void *a, float *c, int32_t *isums, int
 // large problems: 128 x 64 tiles, 4 waves of 64 x 32
 template <Kq T>
 using KqBig = KqConfig<T, 128, 64, 2, 2>;
-// small problems: 32 x 32 tiles. q4_K: 2 waves each taking 2 of the stage's 4
-// sub-blocks (its accuracy bound is per element, so partial super-block sums
-// may be scaled separately). iq2_xxs: one wave, since its bound is per
-// super-block: the integer sum must be complete before it is scaled, or
-// partial sums that nearly cancel would be rounded against a small total.
-template <Kq T>
-using KqTiny = KqConfig<T, 32, 32, 1, 1, T == Kq::Q4K ? 2 : 1>;
-// decode batches: the Tiny tile with 4 or 2 slices of whole super-blocks, so
-// that a few hundred output tiles still keep several waves on every CU (the
-// slices split the K range at super-block boundaries, which the iq2_xxs bound
-// allows)
+// 32 x 32 tiles with 4 or 2 slices of whole super-blocks (the slices split the K
+// range at super-block boundaries, which the iq2_xxs bound allows). q4_K: each
+// slice is 2 waves taking 2 of the stage's 4 sub-blocks (its accuracy bound is
+// per element, so partial super-block sums may be scaled separately). iq2_xxs:
+// one wave, since its bound is per super-block: the integer sum must be complete
+// before it is scaled, or partial sums that nearly cancel would be rounded
+// against a small total.
 template <Kq T>
 using KqMid = KqConfig<T, 32, 32, 1, 1, T == Kq::Q4K ? 2 : 1, 4>;
 template <Kq T>
@@ -733,7 +729,7 @@ using KqBigS2 = KqConfig<T, 128, 64, 2, 2, 1, 2>;
 template <Kq T>
 using KqSmallS2 = KqConfig<T, 64, 64, 2, 2, 1, 2>;
 
-enum { kCfgBig = 0, kCfgTiny = 2, kCfgMid = 3, kCfgMid2 = 4, kCfgBigS2 = 5, kCfgSmallS2 = 6, kCfgWhole = 7, kCfgTiles = 8 };
+enum { kCfgBig = 0, kCfgBigS2 = 1, kCfgSmallS2 = 2, kCfgMid2 = 3, kCfgMid = 4, kCfgGemmTiles = 5, kCfgWhole = 5, kCfgTiles = 6 };
 
 int64_t tiles_of(int64_t m, int64_t n, int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
 
@@ -743,55 +739,85 @@ hipError_t dispatch(const void *w, const void *a, float *c, const MfmaPlan &plan
     switch (plan.config) {
     case kCfgBig: return launch_kq<KqBig<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgMid: return launch_kq<KqMid<T>, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgMid2: return launch_kq<KqMid2<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgBigS2: return launch_kq<KqBigS2<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgSmallS2: return launch_kq<KqSmallS2<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgWhole: return launch_q4_K_small(w, a, c, m, n, k, stream);
     case kCfgTiles:
         return launch_kquant_gemv(T == Kq::Q4K ? PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K : PFNG_WEIGHT_IQ2_XXS_ACTIVATION_Q8_K,
                                   w, a, c, m, n, k, stream);
-    default: return launch_kq<KqTiny<T>, false>(w, a, c, nullptr, m, n, k, stream);
+    default: return launch_kq<KqMid2<T>, false>(w, a, c, nullptr, m, n, k, stream);
+    }
+}
+
+// Predicted time of a tile beyond the launch in nanoseconds, by rounds of one
+// tile per CU (the one-slice 128 x 64 and the two-slice 32 x 32 tiles run two
+// workgroups per CU), fitted to 19 shapes of each format with each tile forced (m
+// 37..2048, n 1000..14336, k 512..11008; mostly within 8 %). us at k = 4096, one
+// round, q4_K / iq2_xxs: 32 x 32 with 4 slices 12.6 / 13.7, with 2 13.6 / 16.5 (two
+// rounds 19.5 / 18.6), 64 x 64 24.2 / 20.6, 128 x 64 with 2 slices 32 / 26.
+int64_t kq_tile_ns(bool q4k, int config, int64_t m, int64_t n, int64_t k, int cus) {
+    auto rounds = [&](int64_t bm, int64_t bn) { return (tiles_of(m, n, bm, bn) + cus - 1) / cus; };
+    const int64_t r64 = rounds(64, 64), r128 = rounds(128, 64), r32 = rounds(32, 32);
+    switch (config) {
+    case kCfgBig:
+        return q4k ? r128 / 2 * (2600 + 135 * k / 10) + r128 % 2 * (1900 + 82 * k / 10)
+                   : r128 / 2 * (2300 + 116 * k / 10) + r128 % 2 * (2000 + 69 * k / 10);
+    case kCfgBigS2: return r128 * (q4k ? 2400 + 69 * k / 10 : 2600 + 56 * k / 10);
+    case kCfgSmallS2: return r64 * (q4k ? 1300 + 48 * k / 10 : 1500 + 425 * k / 100);
+    case kCfgMid2:
+        return q4k ? 1000 + 26 * k / 10 + (r32 - 1) * (400 + 16 * k / 10)
+                   : r32 / 2 * (800 + 39 * k / 10) + r32 % 2 * (1500 + 315 * k / 100);
+    default: return r32 * (1500 + (q4k ? 22 : 25) * k / 10);
     }
 }
 
 }  // namespace
 
-// Tile choice (measured on MI355X, 256 CUs, n = 4096 and the baseline
-// shapes): the 16-row tiles of gemv_kquant.hip for the small m they win
-// (kquant_tiles_as_gemm); q4_K at k = 1024 or 1536 with half to one 32 x 96 tile per CU: the
-// whole-K tiles of gemm_small.hip (c2: 7.60 against 8.59 us for the 64 x 64
-// tiles with 2 slices); 128 x 64 tiles at two or more per CU; with 2
-// super-block slices at one or more per CU (c3); 64 x 64 tiles with 2 slices
-// from half a tile per CU (q4_K) or three quarters (iq2_xxs) (c2 before the
-// whole-K tiles: 9.1 instead of 11.3 us); below that the 32 x 32 tile with the
-// most slices (4, 2, 1) that keeps the waves at or under 8 per CU (more slices
-// only added barrier and staging work). The block-sum diagnostic of the
-// whole-K and the 16-row plans reports the 64 x 64 two-slice tiles' sums (the
-// whole-K tiles split super-blocks between K slices and add the parts only in
-// fp32).
-MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus) {
-    MfmaPlan p;
+// Tile choice: the least predicted time among the tiles with at least `slices`
+// super-block slices (a later one only if it is 3 % less). slices keeps the fp32
+// sums no longer than the tile counts that chose before made them: 1 from two
+// 128 x 64 tiles per CU, 2 from one or from half (q4_K) or three quarters
+// (iq2_xxs) of a 64 x 64 tile per CU, below that 4 while the 32 x 32 tiles' waves
+// stay at 8 per CU; with up to four super-blocks any. us before and now: q4_K
+// 333x4096x4096 43.5 -> 31.8, 333x4096x1536 19.9 -> 14.6, iq2_xxs 333x4096x4096 38.1
+// -> 26.4, 333x1536x4096 33.2 -> 19.7, 333x4096x1536 18.3 -> 12.7.
+int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, int &config) {
     const int64_t c = cus;
     const bool q4k = type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K;
-    const int64_t wk = q4k ? 2 : 1;  // KqTiny's K-waves
     const int64_t t32 = tiles_of(m, n, 32, 32), t64 = tiles_of(m, n, 64, 64), t128 = tiles_of(m, n, 128, 64);
+    int slices = 2;
+    if (k <= 4 * 256 || t128 >= 2 * c)
+        slices = 1;
+    else if (t128 < c && 4 * t64 < (q4k ? 2 : 3) * c && t32 * (q4k ? 8 : 4) <= 8 * c)
+        slices = 4;
+    int64_t best = 0;
+    config = -1;
+    for (int i = kCfgBig; i < kCfgGemmTiles; ++i) {
+        if ((i == kCfgBig ? 1 : i == kCfgMid ? 4 : 2) < slices) continue;
+        const int64_t ns = kq_tile_ns(q4k, i, m, n, k, cus);
+        if (config < 0 || ns + ns * 3 / 100 < best) {
+            best = ns;
+            config = i;
+        }
+    }
+    return best;
+}
+
+// q4_K at k = 1024 or 1536 with half to one 32 x 96 tile per CU takes the whole-K
+// tiles of gemm_small.hip (c2: 7.60 against 8.59 us for the 64 x 64 tiles); small
+// m the 16-row tiles of gemv_kquant.hip where kquant_tiles_as_gemm says so. The
+// block-sum diagnostic of these two plans reports the 64 x 64 two-slice tiles'
+// sums (the whole-K tiles split super-blocks between K slices and add the parts
+// only in fp32).
+MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus) {
+    MfmaPlan p;
     const int64_t t96 = tiles_of(m, n, 32, 96);
     if (kquant_tiles_as_gemm(type, m, n, k, cus))
         p.config = kCfgTiles;
-    else if (q4k && q4_K_small_supported(k) && 2 * t96 >= c && t96 <= c)
+    else if (type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K && q4_K_small_supported(k) && 2 * t96 >= cus && t96 <= cus)
         p.config = kCfgWhole;
-    else if (t128 >= 2 * c)
-        p.config = kCfgBig;
-    else if (t128 >= c)
-        p.config = kCfgBigS2;
-    else if (4 * t64 >= (q4k ? 2 : 3) * c)
-        p.config = kCfgSmallS2;
-    else if (t32 * 4 * wk <= 8 * c)
-        p.config = kCfgMid;
-    else if (t32 * 2 * wk <= 8 * c)
-        p.config = kCfgMid2;
     else
-        p.config = kCfgTiny;
+        best_kquant_tile(type, m, n, k, cus, p.config);
     return p;
 }
 
@@ -819,8 +845,7 @@ hipError_t dispatch_isums(const void *w, const void *a, int32_t *out, const Mfma
     case kCfgTiles:
     case kCfgWhole: return launch_kq<KqIsums<KqSmallS2<T>>, true>(w, a, nullptr, out, m, n, k, stream);
     case kCfgMid: return launch_kq<KqIsums<KqMid<T>>, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgMid2: return launch_kq<KqIsums<KqMid2<T>>, true>(w, a, nullptr, out, m, n, k, stream);
-    default: return launch_kq<KqIsums<KqTiny<T>>, true>(w, a, nullptr, out, m, n, k, stream);
+    default: return launch_kq<KqIsums<KqMid2<T>>, true>(w, a, nullptr, out, m, n, k, stream);
     }
 }
 

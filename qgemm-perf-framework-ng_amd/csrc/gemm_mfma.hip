@@ -612,21 +612,37 @@ bool mfma_supported(int type, int64_t m, int64_t k) {
     return (type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K || type == PFNG_WEIGHT_IQ2_XXS_ACTIVATION_Q8_K) && k % 256 == 0;
 }
 
-// The tile GEMV (16 weight rows a workgroup, one workgroup per CU) repeats its
-// activation chunks in every round, so on wide outputs the GEMM tiles overtake
-// it from m = 17. Its time, by rounds of 16-row tiles and chunks C = m / 16: 1.7
-// us + rounds (2.0 + 1.5 C) (0.25 + 0.75 k / 4096) us. At k = 4096, us GEMV / GEMM:
-// n = 11008 m = 16 12.0 / 12.8, m = 37 20.4 / 17.2, m = 64 24.2 / 17.7, m = 100 36.3 /
-// 27.6; n = 14336 m = 37 29.1 / 17.7, m = 64 33.7 / 18.4, m = 100 49.2 / 28.9. A single
-// round (n <= 4096) keeps the GEMV: m = 64 9.9 / 11.1, m = 100 13.7 / 13.5.
-bool mfma_preferred(int type, int64_t m, int64_t n, int64_t k) {
-    if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 || m <= 16) return false;
-    const int64_t rounds = (n + 16 * kMi355xCus - 1) / (16 * kMi355xCus);
-    if (rounds < 2) return false;
-    const int64_t chunks = (m + 15) / 16;
-    const int64_t gemv = 1700 + rounds * (2000 + 1500 * chunks) * (1024 + 3 * k / 4) / 4096;
+// Rounds of 16-row tiles, one per CU, each repeating its activation chunks C =
+// m / 16: measured at n = 4096 (one round) and m = 16, 37, 64, 100, 128, k = 4096 and
+// 11008, us q4_0 5.2, 8.3, 9.9, 13.7, 15.6, q4_K 5.1, 7.7, 9.6, 13.2, 15.2, iq2_xxs 4.8,
+// 6.6, 7.4, 11.2, 12.6 at k = 4096.
+int64_t tile_gemv_ns(int type, int64_t m, int64_t n, int64_t k, int cus) {
+    const int64_t rounds = (n + 16 * (int64_t)cus - 1) / (16 * (int64_t)cus), chunks = (m + 15) / 16;
+    const int64_t round = type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0   ? 2000 + 1500 * chunks
+                          : type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K ? 1900 + 1430 * chunks
+                                                                     : 1800 + 1120 * chunks;
+    return 1700 + rounds * round * (1024 + 3 * k / 4) / 4096;
+}
+
+int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus) {
     int config;
-    return 2000 + best_q4_0_tile(m, n, k, kMi355xCus, config) < gemv;
+    return 2000 + (type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 ? best_q4_0_tile(m, n, k, cus, config)
+                                                            : best_kquant_tile(type, m, n, k, cus, config));
+}
+
+// The tile GEMV repeats its activation chunks in every round, so on wide outputs
+// the GEMM tiles overtake it from m = 17. At k = 4096, us GEMV / GEMM: q4_0 n = 11008
+// m = 16 12.0 / 12.8, m = 37 20.4 / 17.2, m = 64 24.2 / 17.3, m = 100 35.6 / 27.8; n =
+// 14336 m = 37 29.1 / 17.7, m = 64 33.7 / 18.4; q4_K n = 11008 m = 100 33.9 / 31.3, n =
+// 14336 m = 64 32.6 / 25.5; iq2_xxs n = 11008 m = 128 35.2 / 27.9, n = 14336 m = 64 27.3 /
+// 21.5. A single round (n <= 4096) keeps the GEMV: q4_0 m = 64 9.9 / 11.1. The
+// K-quant GEMM tiles add a slice's super-blocks in one sum, which from about 16
+// of them (k = 8192) is less exact than the GEMV's 16 waves (k = 14336: 1.18e-7
+// against 1.08e-7 from 64 bits), so longer rows stay there.
+bool mfma_preferred(int type, int64_t m, int64_t n, int64_t k) {
+    if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 && k > 8192) return false;
+    return m > 16 && n > 16 * kMi355xCus &&
+           gemm_ns(type, m, n, k, kMi355xCus) < tile_gemv_ns(type, m, n, k, kMi355xCus);
 }
 
 MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus) {

@@ -1569,15 +1569,13 @@ bool kquant_gemv_chunked_fits(int type, int64_t m, int64_t k) {
 // Against the GEMM tiles (us, tiles of 16 weight rows / GEMM): q4_K k = 11008,
 // n = 4096, m = 16 9.4 / 23.4, m = 37 15.2 / 25.4, m = 64 20.1 / 26.5, m = 100
 // 29.5 / 55.1, m = 128 35.4 / 56.9; iq2_xxs m = 16 9.5 / 29.0, m = 100 26.9 /
-// 59.3, m = 128 31.2 / 59.8. Their time goes with the rounds of 16-row tiles, one
-// per CU, so wide outputs from m = 17 stay with the GEMM: k = 2304, n = 11008 (3
-// rounds) m = 100 q4_K 23.6 / 29.5, iq2_xxs 22.8 / 26.2, but n = 14336 (4 rounds)
-// 30.9 / 29.8 and 29.9 / 26.4; k = 1280 q4_K n = 8192 (2 rounds) m = 64 9.8 /
-// 11.3, n = 11008 14.0 / 11.6.
+// 59.3, m = 128 31.2 / 59.8; on wide outputs from m = 17 the GEMM may be faster, as
+// the predicted times say (k = 2304, n = 14336, m = 100: q4_K 30.9 / 29.8, iq2_xxs
+// 29.9 / 26.4).
 bool kquant_tiles_as_gemm(int type, int64_t m, int64_t n, int64_t k, int cus) {
     if (m < kq_tiles_min_m(type, k) || m > gemv_tiles_max_m(k)) return false;
     if (kq_tiles_take_k(type, k) || !kq_tiles_take(type, n, k)) return false;
-    return m <= 16 || (n + 15) / 16 <= (int64_t)cus * (k >= 2048 ? 3 : 2);
+    return m <= 16 || tile_gemv_ns(type, m, n, k, cus) <= gemm_ns(type, m, n, k, cus);
 }
 
 hipError_t launch_kquant_gemv(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,

@@ -59,6 +59,9 @@ struct MfmaPlan {
 
 // gemm_mfma.hip
 bool mfma_supported(int type, int64_t m, int64_t k);
+// predicted times (nanoseconds) of the 16-row tile GEMVs and of the GEMM tiles
+int64_t tile_gemv_ns(int type, int64_t m, int64_t n, int64_t k, int cus);
+int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus);
 // of a shape both tiled paths take: whether the automatic path runs the GEMM
 bool mfma_preferred(int type, int64_t m, int64_t n, int64_t k);
 MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus);
@@ -80,6 +83,8 @@ hipError_t launch_q4_K_small(const void *w, const void *a, float *c, int64_t m, 
                              hipStream_t stream);
 
 // gemm_kquant.hip — q4_K and iq2_xxs against q8_K
+// the GEMM tile with the least predicted time (nanoseconds beyond the launch)
+int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, int &config);
 MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus);
 hipError_t launch_kquant_mul_mat(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                                  const MfmaPlan &plan, hipStream_t stream);

@@ -30,3 +30,23 @@ def test_any_k_bit_exact(hip, torch_gpu, oracle, qtype, m, n, k):
     got = hip.mul_mat(qtype, dev(torch, w), dev(torch, aq), m, n, k)
     torch.cuda.synchronize()
     assert_bits_equal(got.cpu().numpy(), oracle.matmul(qtype, w, aq, m, n, k), f"{m}x{n}x{k} (|a| <= {r})")
+
+
+# the shapes whose tile the predicted times choose: one round of 128x64 two-slice
+# tiles instead of two of 64x64, one-slice tiles at short k, 64x64 instead of 32x32,
+# and wide outputs of 17..128 rows on the GEMM, ragged edges included
+PLAN_CASES = [(q, m, n, k) for q in (1, 2)
+              for m, n, k in [(333, 4090, 512), (330, 1530, 2048), (600, 4001, 768), (130, 600, 1280),
+                              (100, 11000, 256), (37, 14330, 1024), (65, 6100, 2048), (128, 4200, 2304)]]
+
+
+@pytest.mark.parametrize("qtype,m,n,k", PLAN_CASES, ids=[f"{c[0]}-{c[1]}x{c[2]}x{c[3]}" for c in PLAN_CASES])
+def test_planned_tiles_bit_exact(hip, torch_gpu, oracle, qtype, m, n, k):
+    torch = torch_gpu
+    say(f"exact plan type={qtype} {m}x{n}x{k}")
+    _, aq, w, r, _ = exact_case(oracle, qtype, m, n, k, seed=m + n + k + qtype)
+    got = hip.mul_mat(qtype, dev(torch, w), dev(torch, aq), m, n, k)
+    torch.cuda.synchronize()
+    rows = np.unique(np.r_[0, m - 1, np.random.default_rng(m).choice(m, 14, replace=False)])
+    expect = oracle.matmul(qtype, w, np.ascontiguousarray(aq[rows]), len(rows), n, k)
+    assert_bits_equal(got.cpu().numpy()[rows], expect, f"{m}x{n}x{k} (|a| <= {r})")
