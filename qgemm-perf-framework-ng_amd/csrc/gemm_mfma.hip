@@ -638,11 +638,14 @@ int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus) {
 // 21.5. A single round (n <= 4096) keeps the GEMV: q4_0 m = 64 9.9 / 11.1. The
 // K-quant GEMM tiles add a slice's super-blocks in one sum, which from about 16
 // of them (k = 8192) is less exact than the GEMV's 16 waves (k = 14336: 1.18e-7
-// against 1.08e-7 from 64 bits), so longer rows stay there.
+// against 1.08e-7 from 64 bits), so longer rows stay there. A partly filled last
+// round of the GEMV takes less than a whole one, so near a tie the GEMV is the
+// faster one (q4_K 38x13594x8192, predicted 45.0 / 42.6, takes 41.1 / 44.1): the
+// GEMM has to be predicted 7 % faster (100x11008x4096, 37.4 / 34.7, takes 33.9 / 31.3).
 bool mfma_preferred(int type, int64_t m, int64_t n, int64_t k) {
     if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 && k > 8192) return false;
     return m > 16 && n > 16 * kMi355xCus &&
-           gemm_ns(type, m, n, k, kMi355xCus) < tile_gemv_ns(type, m, n, k, kMi355xCus);
+           gemm_ns(type, m, n, k, kMi355xCus) * 107 / 100 < tile_gemv_ns(type, m, n, k, kMi355xCus);
 }
 
 MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus) {
