@@ -94,11 +94,12 @@ __global__ __launch_bounds__(64) void quantize_q4_0_kernel(const float *__restri
     float v[32];
     load_rows32(x, first, nblocks, buf, lane, v);
     // first element of largest magnitude (the reference's strict "<" scan from
-    // 0): the maximum or the minimum, by a scan only where they tie
+    // 0): the maximum or the minimum, by a scan only where they tie or are NaN
+    // (a block of NaNs, which the reference's scan passes over)
     float lo, hi;
     min_max32(v, lo, hi);
     float smax = hi > -lo ? hi : lo;
-    if (__any(!(hi != -lo))) {
+    if (__any(!(hi > -lo || hi < -lo))) {
         float amax = 0.0f, first_max = 0.0f;
 #pragma unroll
         for (int i = 0; i < 32; ++i) {

@@ -69,6 +69,41 @@ def test_values(hip, torch_gpu, oracle, qtype):
     assert bad.size == 0, f"rows {bad} differ"
 
 
+def test_q4_0_infinite_and_nan(hip, torch_gpu, oracle):
+    """Blocks of NaNs, and of NaNs or infinities beside finite values: the scan
+    for the largest magnitude passes over NaN, so a block of 32 NaNs keeps the
+    initial 0 (scale -0), whether the other blocks of its wave (64 blocks)
+    have a tie of magnitudes (an all-zero block does) or not."""
+    torch = torch_gpu
+    nan, inf = np.float32(np.nan), np.float32(np.inf)
+    plain = np.random.default_rng(11).standard_normal((64, 32)).astype(np.float32)
+    plain[:, 5] = 9.0  # one largest magnitude per block: no ties
+    cases = {"one all-NaN block": np.full((1, 32), nan)}
+    for name, rows in {"all-NaN blocks, no tie in the wave": {17: nan, 40: -nan},
+                       "an all-NaN block beside a zero block": {17: nan, 40: 0.0}}.items():
+        x = plain.copy()
+        for r, v in rows.items():
+            x[r] = v
+        cases[name] = x
+    x = plain.copy()
+    x[3, 0] = nan  # the first value
+    x[4, 5] = nan  # the largest
+    x[5, 1:] = nan  # all but one
+    x[6] = nan
+    x[6, 31] = -2.5
+    x[7, 9] = inf
+    x[8, 9] = -inf
+    x[9, [9, 20]] = inf, -inf
+    x[10, [9, 20]] = -inf, inf
+    x[11, [9, 20]] = nan, -inf
+    cases["NaN and infinities beside finite values"] = x
+    for name, x in cases.items():
+        say(f"q4_0 inf / nan: {name}")
+        got = hip.quantize_weights_gpu(0, dev(torch, x)).cpu().numpy().reshape(-1, 18)
+        bad = np.flatnonzero((got != expected(oracle, 0, x).reshape(-1, 18)).any(1))
+        assert bad.size == 0, f"{name}: blocks {bad} differ"
+
+
 def test_q4_K_infinite_and_nan(hip, torch_gpu, oracle):
     """A super-block with an infinite value (its range, and so every quotient,
     leaves the correction steps' bounds) or a NaN beside finite values."""
