@@ -37,6 +37,7 @@
 
 #include "device_common.h"
 #include "kernels.h"
+#include "load_offsets.h"
 
 namespace pfng {
 
@@ -103,11 +104,13 @@ struct PieceRegs {
 };
 
 // What a thread needs of its pieces. Piece p of an operand lies p * kActRows
-// (kWRows) rows below piece 0 in memory and in LDS, so one offset serves all:
-// the row step and the stage go into the loads' uniform offset. Rows past the
-// matrix edge read zeros (the buffer resources are bounded); their results are
-// not stored. BM * nb * 34 < 2^32 for every k up to kMaxTiledK (mfma_supported
-// declines longer rows).
+// (kWRows) rows below piece 0 in memory and in LDS, so one offset serves all,
+// plus the row step (one addition per piece). Rows past the matrix edge read
+// zeros (the buffer resources end at the edge, and the row is part of the lane
+// offset, so they are out of range whether or not the check counts the uniform
+// offset, which only carries the stage); their results are not stored.
+// BM * nb * 34 < 2^32 for every k up to kMaxTiledK (mfma_supported declines
+// longer rows).
 // Consecutive lanes take consecutive pieces of a row, so a wave's load covers
 // whole runs of a few rows (a lane per block pair, as before, touched 32 rows
 // per load, and the address coalescer, not the VALU, set the staging's cost).
@@ -117,13 +120,11 @@ struct PieceRegs {
 // the five dwords from the one at or before its block (half), none of which
 // lies past the block pair's end.
 // Where nb is not a multiple of KB, the last stage's loads of blocks past the
-// row's end are sent out of the resource (to kPastEnd: the largest, 128 rows of
-// 2^24 elements, ends below it) and read zeros: a zero scale on both sides, so
-// such a block adds S * 0.
-constexpr uint32_t kPastEnd = 0xf0000000u;
+// row's end are sent out of the resource (to kPastEnd) and read zeros: a zero
+// scale on both sides, so such a block adds S * 0.
 struct StageSlots {
     uint32_t a, w;               // load offsets of piece 0
-    uint32_t a_last, w_last;     // the same in the last stage: kPastEnd where its block lies past the row
+    uint32_t a_past, w_past;     // kPastEnd where its block lies past the row in the last stage, else 0
     uint32_t sel_a, sel_w;       // v_perm selectors: bytes [2, 6) or [4, 8) of a dword pair
     uint32_t ad_shift, wd_mask;  // the scale's place in dword 0
     int aq, ad, ad_step, wq, wd; // LDS places of piece 0, within a stage buffer
@@ -135,12 +136,12 @@ __device__ __forceinline__ StageSlots stage_slots(int nb) {
     StageSlots o;
     const int ra = threadIdx.x / C::kActPerRow, pa = threadIdx.x % C::kActPerRow;
     const int ja = pa >> 1, ha = pa & 1;
-    o.a = (uint32_t)ra * (uint32_t)nb * 34u + ((34u * (uint32_t)ja + 16u * (uint32_t)ha) & ~3u);
+    o.a = q4_0_act_piece(ra, pa, nb);
     const int rw = threadIdx.x / C::kWPerRow, jw = threadIdx.x % C::kWPerRow;
-    o.w = (uint32_t)rw * (uint32_t)nb * 18u + ((18u * (uint32_t)jw) & ~3u);
+    o.w = q4_0_weight_piece(rw, jw, nb);
     const int tail = nb % C::kKB;
-    o.a_last = tail && ja >= tail ? kPastEnd : o.a;
-    o.w_last = tail && jw >= tail ? kPastEnd : o.w;
+    o.a_past = tail && ja >= tail ? kPastEnd : 0u;
+    o.w_past = tail && jw >= tail ? kPastEnd : 0u;
     o.sel_a = ja & 1 ? kOdd : kEven;
     o.sel_w = jw & 1 ? kOdd : kEven;
     o.ad_shift = ja & 1 ? 16 : 0;
@@ -154,11 +155,11 @@ __device__ __forceinline__ StageSlots stage_slots(int nb) {
     return o;
 }
 
-__device__ __forceinline__ void load5(__amdgpu_buffer_rsrc_t r, uint32_t voffset, uint32_t soffset, uint32_t (&v)[5]) {
-    const i32x4 x = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voffset, soffset, 0));
+__device__ __forceinline__ void load5(__amdgpu_buffer_rsrc_t r, BufferOffset o, uint32_t (&v)[5]) {
+    const i32x4 x = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, o.lane, o.uniform, 0));
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = (uint32_t)x[i];
-    v[4] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, voffset + 16u, soffset, 0);
+    v[4] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, o.lane + 16u, o.uniform, 0);
 }
 
 // Load / store of piece p (activation pieces first). kb: the stage's first
@@ -166,11 +167,16 @@ __device__ __forceinline__ void load5(__amdgpu_buffer_rsrc_t r, uint32_t voffset
 template <class C>
 __device__ __forceinline__ void load_piece(__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rw, const StageSlots &o,
                                            int nb, int kb, bool last, int p, PieceRegs &r) {
-    if (p < C::kActPT)
-        load5(ra, last ? o.a_last : o.a, (uint32_t)(p * C::kActRows) * (uint32_t)nb * 34u + (uint32_t)kb * 34u, r.v);
+    const uint32_t mask = last ? kPastEnd : 0u;
+    const bool act = p < C::kActPT;
+    // opaque, so that the sums with the lane offsets are not kept in a register per piece
+    uint32_t step = act ? (uint32_t)(p * C::kActRows) * (uint32_t)nb * 34u
+                        : (uint32_t)((p - C::kActPT) * C::kWRows) * (uint32_t)nb * 18u;
+    asm volatile("" : "+s"(step));
+    if (act)
+        load5(ra, q4_0_stage_piece(o.a, step, kb * 34, o.a_past & mask), r.v);
     else
-        load5(rw, last ? o.w_last : o.w,
-              (uint32_t)((p - C::kActPT) * C::kWRows) * (uint32_t)nb * 18u + (uint32_t)kb * 18u, r.v);
+        load5(rw, q4_0_stage_piece(o.w, step, kb * 18, o.w_past & mask), r.v);
 }
 
 template <class C>
