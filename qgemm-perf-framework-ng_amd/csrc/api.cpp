@@ -124,10 +124,10 @@ int noalloc_scratch(void **ptr) {
 }
 
 int launch_mfma(int type, const void *weight, const void *act_q, float *out, int64_t m, int64_t n, int64_t k,
-                hipStream_t s) {
+                bool automatic, hipStream_t s) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail(PFNG_ERR_HIP, "hipGetDevice failed");
-    const pfng::MfmaPlan plan = pfng::plan_mfma(type, m, n, k, device_cus(dev));
+    const pfng::MfmaPlan plan = pfng::plan_mfma(type, m, n, k, device_cus(dev), automatic);
     return hip_status(pfng::launch_mfma_mul_mat(type, weight, act_q, out, m, n, k, plan, s), "mfma launch");
 }
 
@@ -214,7 +214,7 @@ int pfng_hip_mul_mat(int type, const void *weight, const void *act_q, float *out
         // may ask for PFNG_PATH_NAIVE explicitly.
         if (gemv_ok && !(mfma_ok && pfng::mfma_preferred(type, m, n, k)))
             return hip_status(pfng::launch_gemv(type, weight, act_q, out, m, n, k, s), "gemv launch");
-        if (mfma_ok) return launch_mfma(type, weight, act_q, out, m, n, k, s);
+        if (mfma_ok) return launch_mfma(type, weight, act_q, out, m, n, k, true, s);
         if (!base_aligned)
             return fail(PFNG_ERR_UNSUPPORTED,
                         "%s: the tiled paths need 16-byte aligned weights and activations and a 4-byte aligned C; "
@@ -238,7 +238,7 @@ int pfng_hip_mul_mat(int type, const void *weight, const void *act_q, float *out
                         "%s MFMA path does not take m=%lld k=%lld: %s, k <= %lld, with 16-byte aligned weights and "
                         "activations and a 4-byte aligned C",
                         type_name(type), (long long)m, (long long)k, mfma_rule(type), (long long)pfng::kMaxTiledK);
-        return launch_mfma(type, weight, act_q, out, m, n, k, s);
+        return launch_mfma(type, weight, act_q, out, m, n, k, false, s);
     case PFNG_PATH_NAIVE:
         return hip_status(pfng::launch_naive_mul_mat(type, weight, act_q, out, m, n, k, s), "naive launch");
     default: return fail(PFNG_ERR_INVALID_ARGUMENT, "unknown path %d", path);
@@ -331,7 +331,7 @@ int pfng_hip_block_isums(int type, const void *weight, const void *act_q, int32_
                     (long long)k);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail(PFNG_ERR_HIP, "hipGetDevice failed");
-    const pfng::MfmaPlan plan = pfng::plan_mfma(type, m, n, k, device_cus(dev));
+    const pfng::MfmaPlan plan = pfng::plan_mfma(type, m, n, k, device_cus(dev), false);
     return hip_status(
         pfng::launch_mfma_block_isums(type, weight, act_q, out, m, n, k, plan, static_cast<hipStream_t>(stream)),
         "block_isums launch");

@@ -781,7 +781,7 @@ int64_t kq_tile_ns(bool q4k, int config, int64_t m, int64_t n, int64_t k, int cu
 // stay at 8 per CU; with up to four super-blocks any. us before and now: q4_K
 // 333x4096x4096 43.5 -> 31.8, 333x4096x1536 19.9 -> 14.6, iq2_xxs 333x4096x4096 38.1
 // -> 26.4, 333x1536x4096 33.2 -> 19.7, 333x4096x1536 18.3 -> 12.7.
-int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, int &config) {
+int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, bool /*automatic*/, int &config) {
     const int64_t c = cus;
     const bool q4k = type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K;
     const int64_t t32 = tiles_of(m, n, 32, 32), t64 = tiles_of(m, n, 64, 64), t128 = tiles_of(m, n, 128, 64);
@@ -809,7 +809,7 @@ int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, int
 // block-sum diagnostic of these two plans reports the 64 x 64 two-slice tiles'
 // sums (the whole-K tiles split super-blocks between K slices and add the parts
 // only in fp32).
-MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus) {
+MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic) {
     MfmaPlan p;
     const int64_t t96 = tiles_of(m, n, 32, 96);
     if (kquant_tiles_as_gemm(type, m, n, k, cus))
@@ -817,7 +817,7 @@ MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus) {
     else if (type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K && q4_K_small_supported(k) && 2 * t96 >= cus && t96 <= cus)
         p.config = kCfgWhole;
     else
-        best_kquant_tile(type, m, n, k, cus, p.config);
+        best_kquant_tile(type, m, n, k, cus, automatic, p.config);
     return p;
 }
 

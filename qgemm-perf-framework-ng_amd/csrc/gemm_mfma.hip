@@ -51,18 +51,19 @@ constexpr uint32_t kBufferWord3 = 0x00020000;  // raw buffer resource
 // AHEAD staging pieces per thread are in flight (a stage has kPieces of them:
 // a deep prefetch for the small tiles, whose stages are too short to cover a
 // memory round trip).
-// FOLD: the accumulators are added into a second set after every two stages, so
-// that no fp32 sum runs over more than a few dozen terms (these tiles take over
-// shapes of the 16-wave tile GEMV, whose sums are that short). It costs no time;
-// relative error from 64 bits on random layers: 100x11008x4096 1.47e-7 without,
-// 9.3e-8 with (9.4e-8 in the tile GEMV), 333x4096x4096 2.0e-7 -> 9.3e-8.
-template <int BM, int BN, int WM, int WN, int KB, int WK = 1, int AHEAD = 6, bool FOLD = false, int MINW = 2>
+// FOLD: the accumulators are added into a second set after every FOLD stages (1 or
+// 2; 0: never), so that no fp32 sum runs over more than a few dozen terms, as in
+// the 16-wave tile GEMV. Relative error from 64 bits on random layers:
+// 100x11008x4096 1.47e-7 without, 9.3e-8 with (9.4e-8 in the tile GEMV),
+// 333x4096x4096 2.0e-7 -> 9.3e-8.
+template <int BM, int BN, int WM, int WN, int KB, int WK = 1, int AHEAD = 6, int FOLD = 0, int MINW = 2>
 struct Q40Config {
     static constexpr int kBM = BM, kBN = BN, kWM = WM, kWN = WN, kKB = KB, kWK = WK, kAhead = AHEAD;
     // waves per SIMD the register budget must allow: the fp32 epilogue needs two
     // resident waves per SIMD to keep the VALU issuing while the other waits
     static constexpr int kMinWavesPerEU = MINW;
-    static constexpr bool kFold = FOLD;
+    static constexpr int kFold = FOLD;
+    using Isums = Q40Config<BM, BN, WM, WN, KB, WK, AHEAD, 0, MINW>;  // of the diagnostic, which folds nothing
     static constexpr int kThreads = 64 * WM * WN * WK;
     static constexpr int kWaveBlocks = KB / WK;  // blocks per stage of one wave
     static constexpr int TM = BM / WM / 32;  // 32x32 tiles per wave along m
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
         for (int j = 0; j < C::TN; ++j) acc[i][j] = (f32x16){};
     f32x16 total[C::TM][C::TN];  // kFold
     auto fold = [&]() __attribute__((always_inline)) {
-        if constexpr (C::kFold && !kIsums) {
+        if constexpr (C::kFold > 0 && !kIsums) {
 #pragma unroll
             for (int i = 0; i < C::TM; ++i)
 #pragma unroll
@@ -385,7 +386,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
                     for (int q = 0; q < 16; ++q) total[i][j][q] += acc[i][j][q];
         }
     };
-    if constexpr (C::kFold && !kIsums) {
+    if constexpr (C::kFold > 0 && !kIsums) {
 #pragma unroll
         for (int i = 0; i < C::TM; ++i)
 #pragma unroll
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
     auto stage = [&](auto R) __attribute__((always_inline)) {
         constexpr int rr = decltype(R)::value;
         __builtin_amdgcn_sched_barrier(0);
-        compute_stage<C, kIsums, C::kFold && rr == 0>(
+        compute_stage<C, kIsums, C::kFold == 1 || (C::kFold == 2 && rr == 0)>(
             lds, rr, acc, isums, m, n, nb, m0, n0, s + rr, tb, lane, wave_m, wave_n,
             [&](int p) __attribute__((always_inline)) {
                 PieceRegs &r = regs[(rr * C::kPieces + p) % C::kAhead];
@@ -446,15 +447,16 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
     };
     for (; s + 1 < stages; s += 2) {
         stage(std::integral_constant<int, 0>{});
+        if constexpr (C::kFold == 1) fold();
         stage(std::integral_constant<int, 1>{});
         fold();
     }
     if (s < stages) {
-        compute_stage<C, kIsums, C::kFold>(lds, 0, acc, isums, m, n, nb, m0, n0, s, tb, lane, wave_m, wave_n,
+        compute_stage<C, kIsums, (C::kFold > 0)>(lds, 0, acc, isums, m, n, nb, m0, n0, s, tb, lane, wave_m, wave_n,
                                            [](int) {});
         fold();
     }
-    if constexpr (C::kFold && !kIsums) {
+    if constexpr (C::kFold > 0 && !kIsums) {
 #pragma unroll
         for (int i = 0; i < C::TM; ++i)
 #pragma unroll
@@ -524,34 +526,65 @@ hipError_t launch_q4_0(const void *w, const void *a, float *c, int32_t *isums, i
 using Q40Big = Q40Config<128, 128, 2, 2, 4, 1, 3>;
 // 128x64, 8 waves of 32x32, 8 blocks per stage (as 4 waves of 64x32 in 2 K-waves
 // it is no faster, and has no registers left to fold into)
-using Q40Mid = Q40Config<128, 64, 4, 2, 8, 1, 5, true>;
+using Q40Mid = Q40Config<128, 64, 4, 2, 8, 1, 5, 2>;
 // 64x64, 4 waves of 32x32 in 2 K-waves each taking 8 of a 16-block stage
-using Q40SmallK2 = Q40Config<64, 64, 2, 2, 16, 2, 6, true>;
+using Q40SmallK2 = Q40Config<64, 64, 2, 2, 16, 2, 6, 2>;
 // 32x64, 2 waves of 32x32 in 4 K-waves each taking 4 of a 16-block stage
-using Q40WideK4 = Q40Config<32, 64, 1, 2, 16, 4, 8, true>;
+using Q40WideK4 = Q40Config<32, 64, 1, 2, 16, 4, 8, 2>;
 // 64x64, 4 waves of 32x32, 8 blocks per stage, two workgroups per CU (short k)
-using Q40Small = Q40Config<64, 64, 2, 2, 8>;
-// 64x64, 2 waves of 64x32, 4 blocks per stage, four workgroups per CU
+using Q40Small = Q40Config<64, 64, 2, 2, 8, 1, 6, 2>;
+// 64x64, 2 waves of 64x32, 4 blocks per stage, four workgroups per CU (no
+// registers left to fold into)
 using Q40Small4 = Q40Config<64, 64, 1, 2, 4>;
 // 32x32, 2 K-waves each taking 4 of an 8-block stage, several workgroups per CU
 // (short k)
-using Q40Tiny = Q40Config<32, 32, 1, 1, 8, 2, 6>;
+using Q40Tiny = Q40Config<32, 32, 1, 1, 8, 2, 6, 2>;
 // 32x32, one wave in 8 K-waves each taking 4 of a 32-block stage, two stages'
 // pieces in flight
-using Q40TinyK8 = Q40Config<32, 32, 1, 1, 32, 8, 12, true>;
+using Q40TinyK8 = Q40Config<32, 32, 1, 1, 32, 8, 12, 2>;
+// The tiles whose wave takes 8 blocks of a stage, folded after every stage: sums
+// of 8 terms, as the tile GEMV has up to k = 4096 (one group per wave and round).
+// us folded every two stages and every one: 126x12859x3584 (128x64) 24.8 / 25.2,
+// 42x15892x2304 (64x64) 12.1 / 12.3. Folding at all costs the 64x64 and 32x32 tiles
+// as much: 906x5111x2816 50.6 / 51.2 (error 1.7e-7 / 8.9e-8), 50x373x1152 6.8 / 6.9
+// (8.4e-8 / 6.7e-8).
+using Q40MidS = Q40Config<128, 64, 4, 2, 8, 1, 5, 1>;
+using Q40SmallK2S = Q40Config<64, 64, 2, 2, 16, 2, 6, 1>;
+using Q40SmallS = Q40Config<64, 64, 2, 2, 8, 1, 6, 1>;
 
 enum {
     kCfgBig = 0,
     kCfgMid = 1,
-    kCfgSmallK2 = 2,
-    kCfgWideK4 = 3,
-    kCfgTinyK8 = 4,
-    kCfgSmall = 5,
-    kCfgTiny = 6,
-    kCfgSmall4 = 7,
-    kCfgTiles = 8,  // the first that is no tile of this file
-    kCfgWhole = 8
+    kCfgMidS = 2,
+    kCfgSmallK2 = 3,
+    kCfgSmallK2S = 4,
+    kCfgWideK4 = 5,
+    kCfgTinyK8 = 6,
+    kCfgSmall = 7,
+    kCfgSmallS = 8,
+    kCfgTiny = 9,
+    kCfgSmall4 = 10,
+    kCfgTiles = 11,  // the first that is no tile of this file
+    kCfgWhole = 11
 };
+
+// f called with the configuration type of a tile of this file
+template <class F>
+auto with_tile(int config, F f) {
+    switch (config) {
+    case kCfgBig: return f(Q40Big{});
+    case kCfgMid: return f(Q40Mid{});
+    case kCfgMidS: return f(Q40MidS{});
+    case kCfgSmallK2: return f(Q40SmallK2{});
+    case kCfgSmallK2S: return f(Q40SmallK2S{});
+    case kCfgWideK4: return f(Q40WideK4{});
+    case kCfgSmall: return f(Q40Small{});
+    case kCfgSmallS: return f(Q40SmallS{});
+    case kCfgTiny: return f(Q40Tiny{});
+    case kCfgSmall4: return f(Q40Small4{});
+    default: return f(Q40TinyK8{});
+    }
+}
 
 int64_t tiles_of(int64_t m, int64_t n, int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
 
@@ -575,9 +608,12 @@ int64_t q4_0_tile_ns(int config, int64_t m, int64_t n, int64_t k, int cus) {
         const int64_t r = rounds(128, 128);
         return r / 2 * (5000 + 198 * k / 10) + r % 2 * (3400 + 135 * k / 10);
     }
-    case kCfgMid: return rounds(128, 64) * (2900 + 575 * padded(256) / 100);
-    case kCfgSmallK2: return rounds(64, 64) * (1700 + 335 * padded(512) / 100);
-    case kCfgSmall: {
+    case kCfgMid:
+    case kCfgMidS: return rounds(128, 64) * (2900 + 575 * padded(256) / 100);
+    case kCfgSmallK2:
+    case kCfgSmallK2S: return rounds(64, 64) * (1700 + 335 * padded(512) / 100);
+    case kCfgSmall:
+    case kCfgSmallS: {
         const int64_t r = rounds(64, 64), p = padded(256);
         return r / 2 * (1600 + 665 * p / 100) + r % 2 * (2200 + 465 * p / 100) * (r > 1 ? 4 : 5) / 5;
     }
@@ -594,18 +630,79 @@ int64_t q4_0_tile_ns(int config, int64_t m, int64_t n, int64_t k, int cus) {
     }
 }
 
+// Rounding (see chain_rounding) of an output's nb block terms in a tile's order:
+// a K-wave adds its blocks one after another, over kFold stages before they go
+// into the total; the K-waves' partials are added in order.
+template <class C>
+int64_t tile_rounding(int64_t nb) {
+    int64_t sum = 0, joined = 0;
+    for (int v = 0; v < C::kWK; ++v) {
+        const int64_t full = nb / C::kKB, rest = nb % C::kKB - v * C::kWaveBlocks;
+        const int64_t terms = full * C::kWaveBlocks + (rest < 0 ? 0 : rest < C::kWaveBlocks ? rest : C::kWaveBlocks);
+        if constexpr (C::kFold > 0) {
+            const int64_t run = C::kFold * C::kWaveBlocks, runs = terms / run, last = terms % run;
+            sum += runs * chain_rounding(run) + chain_rounding(last);
+            if (runs > 0) sum += run * (chain_rounding(runs) - 1) + (last ? terms : 0);
+        } else {
+            sum += chain_rounding(terms);
+        }
+        joined += terms;
+        if (v > 0 && terms > 0) sum += joined;
+    }
+    return sum;
+}
+
+int64_t q4_0_tile_rounding(int config, int64_t nb) {
+    if (config == kCfgWhole) return 4 * chain_rounding(nb / 4) + 9 * (nb / 4);  // four K slices
+    return with_tile(config, [&](auto c) { return tile_rounding<decltype(c)>(nb); });
+}
+
+// The limit of a shape: where the automatic path could run the tile GEMV, that
+// of its 16 waves (8-block groups dealt out in turn); else eight K-waves up to one
+// 32x32 tile per CU, two while there are fewer than two 128x128 and 1.25 64x64 tiles
+// per CU, one sum per output above that and at the k of 4-block stages.
+int64_t q4_0_rounding_limit(int64_t m, int64_t n, int64_t k, int cus, bool automatic) {
+    const int64_t nb = k / 32;
+    if (automatic && m > 16 && gemv_supported(PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0, m, k)) {
+        int64_t sum = 0, joined = 0;
+        for (int v = 0; v < 16 && v < nb / 8; ++v) {
+            const int64_t terms = 8 * ((nb / 8 - v + 15) / 16);
+            sum += chain_rounding(terms);
+            joined += terms;
+            if (v > 0) sum += joined;
+        }
+        return sum;
+    }
+    if (k % 1024 == 0 && tiles_of(m, n, 32, 32) <= cus) return 8 * chain_rounding(nb / 8) + 35 * (nb / 8);
+    if (k % 256 == 0 && tiles_of(m, n, 128, 128) < 2 * (int64_t)cus && 4 * tiles_of(m, n, 64, 64) < 5 * (int64_t)cus)
+        return 2 * chain_rounding(nb / 2) + nb;
+    return chain_rounding(nb);
+}
+
 // The q4_0 tile with the least predicted time (a later one, mostly smaller,
-// only if it is 3 % less).
-int64_t best_q4_0_tile(int64_t m, int64_t n, int64_t k, int cus, int &config) {
-    int64_t best = 0;
+// only if it is 3 % less) among those within the shape's rounding limit. Without
+// the limit, errors from 64 bits against the tile GEMV's: 100x20480x4096
+// (2-wave 64x64) 2.2 times, 48x28672x8192 (64x64) 2.6, 74x10537x3072 (32x32) 1.7.
+int64_t best_q4_0_tile(int64_t m, int64_t n, int64_t k, int cus, bool automatic, int &config) {
+    const int64_t limit = q4_0_rounding_limit(m, n, k, cus, automatic);
+    int64_t best = kNoTile;
+    config = kCfgBig;
     for (int c = kCfgBig; c < kCfgTiles; ++c) {
         const int64_t ns = q4_0_tile_ns(c, m, n, k, cus);
-        if (c == kCfgBig || ns + ns * 3 / 100 < best) {
+        if (ns + ns * 3 / 100 < best && within_rounding(q4_0_tile_rounding(c, k / 32), limit)) {
             best = ns;
             config = c;
         }
     }
     return best;
+}
+
+// Whole-K 32x96 tiles, one per CU and one round (480x1536x1536: 7.0 us against
+// 8.9 us for the 64x64 tile), where their four K slices are within the limit
+bool q4_0_takes_whole(int64_t m, int64_t n, int64_t k, int cus, bool automatic) {
+    const int64_t tiles = tiles_of(m, n, 32, 96);
+    return q4_0_small_supported(k) && 2 * tiles >= cus && tiles <= cus &&
+           within_rounding(q4_0_tile_rounding(kCfgWhole, k / 32), q4_0_rounding_limit(m, n, k, cus, automatic));
 }
 
 }  // namespace
@@ -630,10 +727,12 @@ int64_t tile_gemv_ns(int type, int64_t m, int64_t n, int64_t k, int cus) {
     return 1700 + rounds * round * (1024 + 3 * k / 4) / 4096;
 }
 
-int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus) {
+int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic) {
     int config;
-    return 2000 + (type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 ? best_q4_0_tile(m, n, k, cus, config)
-                                                            : best_kquant_tile(type, m, n, k, cus, config));
+    if (type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 && q4_0_takes_whole(m, n, k, cus, automatic))
+        return 3000 + 26 * k / 10;  // 5.7 us at k = 1024, 7.0 at 1536
+    return 2000 + (type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 ? best_q4_0_tile(m, n, k, cus, automatic, config)
+                                                            : best_kquant_tile(type, m, n, k, cus, automatic, config));
 }
 
 // The tile GEMV repeats its activation chunks in every round, so on wide outputs
@@ -651,53 +750,37 @@ int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus) {
 bool mfma_preferred(int type, int64_t m, int64_t n, int64_t k) {
     if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 && k > 8192) return false;
     return m > 16 && n > 16 * kMi355xCus &&
-           gemm_ns(type, m, n, k, kMi355xCus) * 107 / 100 < tile_gemv_ns(type, m, n, k, kMi355xCus);
+           gemm_ns(type, m, n, k, kMi355xCus, true) * 107 / 100 < tile_gemv_ns(type, m, n, k, kMi355xCus);
 }
 
-MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus) {
-    if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0) return plan_kquant(type, m, n, k, cus);
+MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic) {
+    if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0) return plan_kquant(type, m, n, k, cus, automatic);
     MfmaPlan p;
-    if (q4_0_small_supported(k) && 2 * tiles_of(m, n, 32, 96) >= cus && tiles_of(m, n, 32, 96) <= cus) {
-        // whole-K 32x96 tiles, one per CU and one round (480x1536x1536:
-        // 7.0 us against 8.9 us for the 64x64 tile)
+    if (q4_0_takes_whole(m, n, k, cus, automatic)) {
         p.config = kCfgWhole;
         return p;
     }
-    best_q4_0_tile(m, n, k, cus, p.config);
+    best_q4_0_tile(m, n, k, cus, automatic, p.config);
     return p;
 }
 
 hipError_t launch_mfma_mul_mat(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                                const MfmaPlan &plan, hipStream_t stream) {
     if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0) return launch_kquant_mul_mat(type, w, a, c, m, n, k, plan, stream);
-    switch (plan.config) {
-    case kCfgBig: return launch_q4_0<Q40Big, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgMid: return launch_q4_0<Q40Mid, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgSmallK2: return launch_q4_0<Q40SmallK2, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgWideK4: return launch_q4_0<Q40WideK4, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgSmall: return launch_q4_0<Q40Small, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgTiny: return launch_q4_0<Q40Tiny, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgSmall4: return launch_q4_0<Q40Small4, false>(w, a, c, nullptr, m, n, k, stream);
-    case kCfgWhole: return launch_q4_0_small(w, a, c, nullptr, m, n, k, stream);
-    default: return launch_q4_0<Q40TinyK8, false>(w, a, c, nullptr, m, n, k, stream);
-    }
+    if (plan.config == kCfgWhole) return launch_q4_0_small(w, a, c, nullptr, m, n, k, stream);
+    return with_tile(plan.config, [&](auto t) {
+        return launch_q4_0<decltype(t), false>(w, a, c, nullptr, m, n, k, stream);
+    });
 }
 
 hipError_t launch_mfma_block_isums(int type, const void *w, const void *a, int32_t *out, int64_t m, int64_t n,
                                    int64_t k, const MfmaPlan &plan, hipStream_t stream) {
     if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0)
         return launch_kquant_block_isums(type, w, a, out, m, n, k, plan, stream);
-    switch (plan.config) {
-    case kCfgBig: return launch_q4_0<Q40Big, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgMid: return launch_q4_0<Q40Mid, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgSmallK2: return launch_q4_0<Q40SmallK2, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgWideK4: return launch_q4_0<Q40WideK4, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgSmall: return launch_q4_0<Q40Small, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgTiny: return launch_q4_0<Q40Tiny, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgSmall4: return launch_q4_0<Q40Small4, true>(w, a, nullptr, out, m, n, k, stream);
-    case kCfgWhole: return launch_q4_0_small(w, a, nullptr, out, m, n, k, stream);
-    default: return launch_q4_0<Q40TinyK8, true>(w, a, nullptr, out, m, n, k, stream);
-    }
+    if (plan.config == kCfgWhole) return launch_q4_0_small(w, a, nullptr, out, m, n, k, stream);
+    return with_tile(plan.config, [&](auto t) {
+        return launch_q4_0<typename decltype(t)::Isums, true>(w, a, nullptr, out, m, n, k, stream);
+    });
 }
 
 }  // namespace pfng

@@ -1575,7 +1575,7 @@ bool kquant_gemv_chunked_fits(int type, int64_t m, int64_t k) {
 bool kquant_tiles_as_gemm(int type, int64_t m, int64_t n, int64_t k, int cus) {
     if (m < kq_tiles_min_m(type, k) || m > gemv_tiles_max_m(k)) return false;
     if (kq_tiles_take_k(type, k) || !kq_tiles_take(type, n, k)) return false;
-    return m <= 16 || tile_gemv_ns(type, m, n, k, cus) <= gemm_ns(type, m, n, k, cus);
+    return m <= 16 || tile_gemv_ns(type, m, n, k, cus) <= gemm_ns(type, m, n, k, cus, false);
 }
 
 hipError_t launch_kquant_gemv(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,

@@ -57,14 +57,27 @@ struct MfmaPlan {
     int config = 0;
 };
 
+// How exact a summation order is: the mean square rounding error of an output,
+// in units of one rounding of one term (terms of like size and random sign). A
+// partial sum of i terms is rounded with weight i, so n terms added one after
+// another come to n (n + 1) / 2.
+constexpr int64_t chain_rounding(int64_t n) { return n * (n + 1) / 2; }
+// Whether a tile's sums are as exact as a shape's limit asks (3 % for the
+// model's own error, 1.5 % in the error's size).
+constexpr bool within_rounding(int64_t rounding, int64_t limit) { return rounding <= limit + limit * 3 / 100; }
+// predicted time of a GEMM of which no tile is within its limit
+constexpr int64_t kNoTile = INT64_MAX / 256;
+
 // gemm_mfma.hip
 bool mfma_supported(int type, int64_t m, int64_t k);
-// predicted times (nanoseconds) of the 16-row tile GEMVs and of the GEMM tiles
+// Predicted times (nanoseconds) of the 16-row tile GEMVs and of the GEMM tiles.
+// automatic: the path was not asked for by name, so that a shape which the tile
+// GEMV takes too is to be summed as exactly as there.
 int64_t tile_gemv_ns(int type, int64_t m, int64_t n, int64_t k, int cus);
-int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus);
+int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic);
 // of a shape both tiled paths take: whether the automatic path runs the GEMM
 bool mfma_preferred(int type, int64_t m, int64_t n, int64_t k);
-MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus);
+MfmaPlan plan_mfma(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic);
 hipError_t launch_mfma_mul_mat(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                                const MfmaPlan &plan, hipStream_t stream);
 // the integer block sums of the configuration `plan` selects (diagnostic)
@@ -84,8 +97,8 @@ hipError_t launch_q4_K_small(const void *w, const void *a, float *c, int64_t m, 
 
 // gemm_kquant.hip — q4_K and iq2_xxs against q8_K
 // the GEMM tile with the least predicted time (nanoseconds beyond the launch)
-int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, int &config);
-MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus);
+int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic, int &config);
+MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic);
 hipError_t launch_kquant_mul_mat(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                                  const MfmaPlan &plan, hipStream_t stream);
 hipError_t launch_kquant_block_isums(int type, const void *w, const void *a, int32_t *out, int64_t m, int64_t n,

@@ -22,12 +22,20 @@ CASES = ([(2048, 4096, 128), (2000, 4100, 256), (1921, 4097, 384), (2048, 4096, 
          + [(40, 4100, 4096), (130, 4033, 4224), (500, 4000, 1664), (1000, 1500, 1280)])
 
 
-@pytest.mark.parametrize("m,n,k", CASES, ids=[f"{m}x{n}x{k}" for m, n, k in CASES])
-def test_staging_bit_exact(hip, torch_gpu, oracle, m, n, k):
+# the tiles that fold their sums after every stage (128x64, 64x64 and its two K-waves), which the
+# automatic path takes where two stages' sums would be longer than the tile GEMV's
+AUTO_CASES = [(100, 8327, 2048), (100, 8327, 2304), (500, 1832, 768), (33, 8327, 1536), (100, 4430, 2304),
+              (500, 2265, 512), (500, 2265, 768)]
+
+
+@pytest.mark.parametrize("m,n,k,auto", [(*c, False) for c in CASES] + [(*c, True) for c in AUTO_CASES],
+                         ids=[f"{m}x{n}x{k}" for m, n, k in CASES] + [f"auto-{m}x{n}x{k}" for m, n, k in AUTO_CASES])
+def test_staging_bit_exact(hip, torch_gpu, oracle, m, n, k, auto):
     torch = torch_gpu
     say(f"exact q4_0 staging {m}x{n}x{k}")
     _, aq, w, r, _ = exact_case(oracle, 0, m, n, k, seed=m + n + k)
-    got = hip.mul_mat(0, dev(torch, w), dev(torch, aq), m, n, k, path=hip.PATH_MFMA)
+    assert hip.auto_path(0, m, n, k) == hip.PATH_MFMA or not auto
+    got = hip.mul_mat(0, dev(torch, w), dev(torch, aq), m, n, k, path=hip.PATH_AUTO if auto else hip.PATH_MFMA)
     torch.cuda.synchronize()
     rows = np.unique(np.r_[0, m - 1, np.random.default_rng(m).choice(m, min(m, 24), replace=False)])
     expect = oracle.matmul(0, w, np.ascontiguousarray(aq[rows]), len(rows), n, k)
