@@ -35,6 +35,8 @@
 // VALU work. The split is a byte lookup (v_perm) into a per-scale table of the
 // six (lo, hi) pairs of +-8, +-25, +-43 times the scale.
 // A diagnostic instantiation writes the int32 super-block sums instead of C.
+#include <type_traits>
+
 #include "device_common.h"
 #include "kernels.h"
 #include "pfng_iq2xxs_grid.h"
@@ -51,9 +53,10 @@ enum class Kq { Q4K, IQ2 };
 // stage divided among WK waves, and WS slices of such waves that take every
 // WS-th super-block each (each slice stages its own super-blocks in its own
 // LDS buffers). WK * WS > 1: the partial accumulators are added through LDS
-// at the end, in a fixed order.
-template <Kq T, int BM, int BN, int WM, int WN, int WK = 1, int WS = 1>
+// at the end, in a fixed order and in SUM.
+template <Kq T, int BM, int BN, int WM, int WN, int WK = 1, int WS = 1, class SUM = float>
 struct KqConfig {
+    using Sum = SUM;
     static constexpr Kq kType = T;
     static constexpr bool kQ4K = T == Kq::Q4K;
     static constexpr int kBM = BM, kBN = BN, kWM = WM, kWN = WN, kWK = WK, kWS = WS;
@@ -670,15 +673,17 @@ __global__ __launch_bounds__(C::kAllThreads, 2) void gemm_kq_kernel(const uint8_
             __syncthreads();
             if (grp > 0) return;
 #pragma unroll
-            for (int g2 = 1; g2 < kGroups; ++g2) {
-                const float *src = red + ((g2 - 1) * C::kWM * C::kWN + wmn) * kRegs * 64 + lane;
+            for (int tm = 0; tm < C::TM; ++tm)
 #pragma unroll
-                for (int tm = 0; tm < C::TM; ++tm)
+                for (int tn = 0; tn < C::TN; ++tn)
 #pragma unroll
-                    for (int tn = 0; tn < C::TN; ++tn)
+                    for (int r = 0; r < 16; ++r) {
+                        typename C::Sum s = A.acc[tm][tn][r];
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) A.acc[tm][tn][r] += src[((tm * C::TN + tn) * 16 + r) * 64];
-            }
+                        for (int g2 = 1; g2 < kGroups; ++g2)
+                            s += red[(((g2 - 1) * C::kWM * C::kWN + wmn) * kRegs + (tm * C::TN + tn) * 16 + r) * 64 + lane];
+                        A.acc[tm][tn][r] = (float)s;
+                    }
         }
         const int li = lane & 31;
 #pragma unroll
@@ -721,6 +726,11 @@ template <Kq T>
 using KqMid = KqConfig<T, 32, 32, 1, 1, T == Kq::Q4K ? 2 : 1, 4>;
 template <Kq T>
 using KqMid2 = KqConfig<T, 32, 32, 1, 1, T == Kq::Q4K ? 2 : 1, 2>;
+// q4_K: the four partials of an output added in fp64, which leaves one rounding
+// of the sum instead of three: as exact as two slices of whole super-blocks
+// (24x10674x768 8.3e-8 -> 7.3e-8 from 64 bits), for 0.35 us
+template <Kq T>
+using KqMid2D = KqConfig<T, 32, 32, 1, 1, T == Kq::Q4K ? 2 : 1, 2, std::conditional_t<T == Kq::Q4K, double, float>>;
 
 // the 128 x 64 and 64 x 64 tiles with 2 slices: 8 waves per workgroup where
 // the tiles alone give about one workgroup per CU
@@ -729,7 +739,17 @@ using KqBigS2 = KqConfig<T, 128, 64, 2, 2, 1, 2>;
 template <Kq T>
 using KqSmallS2 = KqConfig<T, 64, 64, 2, 2, 1, 2>;
 
-enum { kCfgBig = 0, kCfgBigS2 = 1, kCfgSmallS2 = 2, kCfgMid2 = 3, kCfgMid = 4, kCfgGemmTiles = 5, kCfgWhole = 5, kCfgTiles = 6 };
+enum {
+    kCfgBig = 0,
+    kCfgBigS2 = 1,
+    kCfgSmallS2 = 2,
+    kCfgMid2 = 3,
+    kCfgMid2D = 4,
+    kCfgMid = 5,
+    kCfgGemmTiles = 6,  // the first that is no tile of this file
+    kCfgWhole = 6,
+    kCfgTiles = 7
+};
 
 int64_t tiles_of(int64_t m, int64_t n, int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
 
@@ -739,6 +759,7 @@ hipError_t dispatch(const void *w, const void *a, float *c, const MfmaPlan &plan
     switch (plan.config) {
     case kCfgBig: return launch_kq<KqBig<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgMid: return launch_kq<KqMid<T>, false>(w, a, c, nullptr, m, n, k, stream);
+    case kCfgMid2D: return launch_kq<KqMid2D<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgBigS2: return launch_kq<KqBigS2<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgSmallS2: return launch_kq<KqSmallS2<T>, false>(w, a, c, nullptr, m, n, k, stream);
     case kCfgWhole: return launch_q4_K_small(w, a, c, m, n, k, stream);
@@ -765,37 +786,69 @@ int64_t kq_tile_ns(bool q4k, int config, int64_t m, int64_t n, int64_t k, int cu
     case kCfgBigS2: return r128 * (q4k ? 2400 + 69 * k / 10 : 2600 + 56 * k / 10);
     case kCfgSmallS2: return r64 * (q4k ? 1300 + 48 * k / 10 : 1500 + 425 * k / 100);
     case kCfgMid2:
-        return q4k ? 1000 + 26 * k / 10 + (r32 - 1) * (400 + 16 * k / 10)
-                   : r32 / 2 * (800 + 39 * k / 10) + r32 % 2 * (1500 + 315 * k / 100);
+    case kCfgMid2D:
+        return (config == kCfgMid2D ? 350 : 0) +
+               (q4k ? 1000 + 26 * k / 10 + (r32 - 1) * (400 + 16 * k / 10)
+                    : r32 / 2 * (800 + 39 * k / 10) + r32 % 2 * (1500 + 315 * k / 100));
     default: return r32 * (1500 + (q4k ? 22 : 25) * k / 10);
     }
 }
 
-}  // namespace
+// Rounding of the super-block sums (see chain_rounding; twice, since a K-wave's
+// part of a super-block counts half): a slice adds its super-blocks one after
+// another, then the slices' and K-waves' partials are added in order, or in fp64.
+// A term has roundings of its own: its product and, for q4_K, those of d * IS and
+// dmin * IM, which are larger than their difference (about 5 in all, from measured
+// errors).
+int64_t kq_rounding(bool q4k, int slices, int waves, bool fp64, int64_t nsb) {
+    int64_t twice = 2 * (q4k ? 5 : 1) * nsb, joined = 0;
+    for (int s = 0; s < slices && s < nsb; ++s) {
+        const int64_t terms = (nsb - s + slices - 1) / slices;
+        twice += 2 * chain_rounding(terms);
+        for (int v = 0; v < waves; ++v) {
+            joined += 2 * terms / waves;
+            if (!fp64 && s + v > 0) twice += joined;
+        }
+    }
+    return twice + (fp64 ? joined : 0);
+}
 
-// Tile choice: the least predicted time among the tiles with at least `slices`
-// super-block slices (a later one only if it is 3 % less). slices keeps the fp32
-// sums no longer than the tile counts that chose before made them: 1 from two
-// 128 x 64 tiles per CU, 2 from one or from half (q4_K) or three quarters
-// (iq2_xxs) of a 64 x 64 tile per CU, below that 4 while the 32 x 32 tiles' waves
-// stay at 8 per CU; with up to four super-blocks any. us before and now: q4_K
-// 333x4096x4096 43.5 -> 31.8, 333x4096x1536 19.9 -> 14.6, iq2_xxs 333x4096x4096 38.1
-// -> 26.4, 333x1536x4096 33.2 -> 19.7, 333x4096x1536 18.3 -> 12.7.
-int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, bool /*automatic*/, int &config) {
+// q4_K whole-K tiles (gemm_small.hip): at k = 1024 or 1536 with half to one 32 x 96
+// tile per CU (c2: 7.60 against 8.59 us for the 64 x 64 tiles)
+bool takes_whole(int type, int64_t m, int64_t n, int64_t k, int cus) {
+    const int64_t tiles = tiles_of(m, n, 32, 96);
+    return type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K && q4_K_small_supported(k) && 2 * tiles >= cus && tiles <= cus;
+}
+
+// Tile choice: the least predicted time (a later tile only if it is 3 % less)
+// among the tiles with at least `slices` super-block slices whose sums are
+// within the shape's rounding limit. slices is 1 from two 128 x 64 tiles per CU,
+// 2 from one or from half (q4_K) or three quarters (iq2_xxs) of a 64 x 64 tile per
+// CU, below that 4 while the 32 x 32 tiles' waves stay at 8 per CU; with up to
+// four super-blocks any. The limit is that of the tile so chosen, or, where the
+// automatic path could run the tile GEMV, of its 16 waves. us
+// with these slices and the fastest: q4_K 333x4096x4096 43.5 -> 31.8,
+// 333x4096x1536 19.9 -> 14.6, iq2_xxs 333x4096x4096 38.1 -> 26.4, 333x1536x4096
+// 33.2 -> 19.7, 333x4096x1536 18.3 -> 12.7.
+int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic, int &config) {
     const int64_t c = cus;
     const bool q4k = type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K;
     const int64_t t32 = tiles_of(m, n, 32, 32), t64 = tiles_of(m, n, 64, 64), t128 = tiles_of(m, n, 128, 64);
-    int slices = 2;
-    if (k <= 4 * 256 || t128 >= 2 * c)
-        slices = 1;
-    else if (t128 < c && 4 * t64 < (q4k ? 2 : 3) * c && t32 * (q4k ? 8 : 4) <= 8 * c)
-        slices = 4;
-    int64_t best = 0;
-    config = -1;
+    const bool one = t128 >= 2 * c, two = t128 >= c || 4 * t64 >= (q4k ? 2 : 3) * c;
+    const bool four = !two && t32 * (q4k ? 8 : 4) <= 8 * c;
+    const int slices = k <= 4 * 256 || one ? 1 : four ? 4 : 2;
+    const int64_t nsb = k / 256;
+    const bool gemv = automatic && m > 16 && gemv_supported(type, m, k);
+    const int waves = q4k ? 2 : 1;  // of the 32 x 32 tiles
+    const int64_t limit = kq_rounding(q4k, gemv ? 16 : one ? 1 : four ? 4 : 2, gemv || one || two ? 1 : waves, false, nsb);
+    int64_t best = kNoTile;
+    config = kCfgBig;
     for (int i = kCfgBig; i < kCfgGemmTiles; ++i) {
-        if ((i == kCfgBig ? 1 : i == kCfgMid ? 4 : 2) < slices) continue;
+        const int ws = i == kCfgBig ? 1 : i == kCfgMid ? 4 : 2;
+        if (ws < slices || (i == kCfgMid2D && !q4k)) continue;
+        if (!within_rounding(kq_rounding(q4k, ws, i >= kCfgMid2 ? waves : 1, i == kCfgMid2D, nsb), limit)) continue;
         const int64_t ns = kq_tile_ns(q4k, i, m, n, k, cus);
-        if (config < 0 || ns + ns * 3 / 100 < best) {
+        if (ns + ns * 3 / 100 < best) {
             best = ns;
             config = i;
         }
@@ -803,18 +856,23 @@ int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, boo
     return best;
 }
 
-// q4_K at k = 1024 or 1536 with half to one 32 x 96 tile per CU takes the whole-K
-// tiles of gemm_small.hip (c2: 7.60 against 8.59 us for the 64 x 64 tiles); small
-// m the 16-row tiles of gemv_kquant.hip where kquant_tiles_as_gemm says so. The
-// block-sum diagnostic of these two plans reports the 64 x 64 two-slice tiles'
-// sums (the whole-K tiles split super-blocks between K slices and add the parts
-// only in fp32).
+}  // namespace
+
+int64_t kquant_gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic) {
+    int config;
+    if (takes_whole(type, m, n, k, cus)) return 3000 + 26 * k / 10;  // 5.5 us at k = 1024, 7.1 at 1536
+    return 2000 + best_kquant_tile(type, m, n, k, cus, automatic, config);
+}
+
+// Small m takes the 16-row tiles of gemv_kquant.hip where kquant_tiles_as_gemm says
+// so. The block-sum diagnostic of these and the whole-K plan reports the 64 x 64
+// two-slice tiles' sums (the whole-K tiles split super-blocks between K slices and
+// add the parts only in fp32).
 MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic) {
     MfmaPlan p;
-    const int64_t t96 = tiles_of(m, n, 32, 96);
     if (kquant_tiles_as_gemm(type, m, n, k, cus))
         p.config = kCfgTiles;
-    else if (type == PFNG_WEIGHT_Q4_K_ACTIVATION_Q8_K && q4_K_small_supported(k) && 2 * t96 >= cus && t96 <= cus)
+    else if (takes_whole(type, m, n, k, cus))
         p.config = kCfgWhole;
     else
         best_kquant_tile(type, m, n, k, cus, automatic, p.config);

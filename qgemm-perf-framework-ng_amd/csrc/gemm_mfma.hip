@@ -728,11 +728,10 @@ int64_t tile_gemv_ns(int type, int64_t m, int64_t n, int64_t k, int cus) {
 }
 
 int64_t gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic) {
+    if (type != PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0) return kquant_gemm_ns(type, m, n, k, cus, automatic);
+    if (q4_0_takes_whole(m, n, k, cus, automatic)) return 3000 + 26 * k / 10;  // 5.7 us at k = 1024, 7.0 at 1536
     int config;
-    if (type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 && q4_0_takes_whole(m, n, k, cus, automatic))
-        return 3000 + 26 * k / 10;  // 5.7 us at k = 1024, 7.0 at 1536
-    return 2000 + (type == PFNG_WEIGHT_Q4_0_ACTIVATION_Q8_0 ? best_q4_0_tile(m, n, k, cus, automatic, config)
-                                                            : best_kquant_tile(type, m, n, k, cus, automatic, config));
+    return 2000 + best_q4_0_tile(m, n, k, cus, automatic, config);
 }
 
 // The tile GEMV repeats its activation chunks in every round, so on wide outputs

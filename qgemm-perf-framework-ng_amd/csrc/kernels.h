@@ -96,8 +96,7 @@ hipError_t launch_q4_K_small(const void *w, const void *a, float *c, int64_t m, 
                              hipStream_t stream);
 
 // gemm_kquant.hip — q4_K and iq2_xxs against q8_K
-// the GEMM tile with the least predicted time (nanoseconds beyond the launch)
-int64_t best_kquant_tile(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic, int &config);
+int64_t kquant_gemm_ns(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic);  // see gemm_ns
 MfmaPlan plan_kquant(int type, int64_t m, int64_t n, int64_t k, int cus, bool automatic);
 hipError_t launch_kquant_mul_mat(int type, const void *w, const void *a, float *c, int64_t m, int64_t n, int64_t k,
                                  const MfmaPlan &plan, hipStream_t stream);
