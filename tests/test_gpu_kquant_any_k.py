@@ -34,10 +34,12 @@ def test_any_k_bit_exact(hip, torch_gpu, oracle, qtype, m, n, k):
 
 # the shapes whose tile the predicted times choose: one round of 128x64 two-slice
 # tiles instead of two of 64x64, one-slice tiles at short k, 64x64 instead of 32x32,
-# and wide outputs of 17..128 rows on the GEMM, ragged edges included
+# wide outputs of 17..128 rows on the GEMM (q4_K also on whole-K tiles), the q4_K 32x32
+# tile whose partials are added in fp64; ragged edges included
 PLAN_CASES = [(q, m, n, k) for q in (1, 2)
               for m, n, k in [(333, 4090, 512), (330, 1530, 2048), (600, 4001, 768), (130, 600, 1280),
-                              (100, 11000, 256), (37, 14330, 1024), (65, 6100, 2048), (128, 4200, 2304)]]
+                              (100, 11000, 256), (37, 14330, 1024), (65, 6100, 2048), (128, 4200, 2304),
+                              (40, 6500, 1024), (333, 1363, 1280), (333, 1363, 2048)]]
 
 
 @pytest.mark.parametrize("qtype,m,n,k", PLAN_CASES, ids=[f"{c[0]}-{c[1]}x{c[2]}x{c[3]}" for c in PLAN_CASES])
