@@ -1084,22 +1084,24 @@ __host__ __device__ constexpr int q4k_chunk_lds_bytes(int c) {
     return kKqMfWaves * kChunkWaveBytes + (c == 1 ? kChunkPartialBytes : 0);
 }
 
-// The 16 waves' partials, kStride floats apart, added in T in pairs (a fixed
+// The first kN waves' partials, kStride floats apart, added in T in pairs (a fixed
 // order). Relative error from 64 bits on random layers against fp32 sums in wave
 // order (k = 4096) or the GEMM tiles' slices (k = 2816): q4_K 1.03e-7 -> 8.7e-8 and
 // 9.1e-8 -> 8.5e-8, iq2_xxs 8.4e-8 -> 6.5e-8 and 6.0e-8 -> 6.3e-8 in fp32; in fp64
-// 7.2e-8, 7.2e-8, 4.3e-8 and 4.3e-8, for 1-2 % of the time (4096 x 4096, m = 128
-// q4_K 15.35 -> 15.49 us). So the iq2_xxs rows that the GEMM slices used to add
-// take fp64, the others fp32, which costs nothing.
-template <int kStride, class T = float>
+// 7.2e-8, 7.2e-8, 4.3e-8 and 4.3e-8, for 1-2 % of the time at n = 4096 (4096 x 4096,
+// m = 128 q4_K 15.35 -> 15.49 us) and up to 8 % on wide outputs (45x20393x1792 17.7
+// -> 19.1). So fp64 is for the rows that GEMM slices would add more exactly than
+// fp32 pairs: iq2_xxs at every such k, q4_K up to 14 super-blocks from m = 17
+// (20x9221x1280 8.5e-8 -> 7.7e-8, two slices 8.0e-8).
+template <int kStride, class T = float, int kN = kKqMfWaves>
 __device__ __forceinline__ float sum_wave_partials(const float *p) {
-    T v[kKqMfWaves];
+    T v[kN];
 #pragma unroll
-    for (int i = 0; i < kKqMfWaves; ++i) v[i] = (T)p[i * kStride];
+    for (int i = 0; i < kN; ++i) v[i] = (T)p[i * kStride];
 #pragma unroll
-    for (int step = 1; step < kKqMfWaves; step *= 2)
+    for (int step = 1; step < kN; step *= 2)
 #pragma unroll
-        for (int i = 0; i < kKqMfWaves; i += 2 * step) v[i] += v[i + step];
+        for (int i = 0; i + step < kN; i += 2 * step) v[i] += v[i + step];
     return (float)v[0];
 }
 
@@ -1232,9 +1234,12 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[wave * kStride + (ch * 4 + r) * 64 + lane] = acc[ch][r];
     __syncthreads();
+    // (one chunk: m <= 16)
+    const bool few = C > 1 && kG == 0 && !even_rows && nsb <= 14;
     const int col = n0 + li;
     for (int g = wave; g < 4 * C; g += kKqMfWaves) {
-        const float s = sum_wave_partials<kStride>(red + g * 64 + lane);
+        const float *p = red + g * 64 + lane;
+        const float s = few ? sum_wave_partials<kStride, double, 14>(p) : sum_wave_partials<kStride>(p);
         const int row = 16 * (g / 4) + 4 * q + g % 4;
         if (col < n && row < m) store_through(&c[(size_t)row * n + col], s);
     }

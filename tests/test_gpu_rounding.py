@@ -32,10 +32,10 @@ def random_weights(torch, qtype, n, k, seed):
     return w.reshape(n, -1)
 
 
-def wave_sums(oracle, qtype, w, aq, m, k):
+def wave_sums(oracle, qtype, w, aq, m, k, waves=16):
     """The product with the rows of w, in 64 bits from the exact block sums, and
-    in fp32 as 16 waves add it: blocks in groups of 256 values dealt out in turn,
-    one fused multiply-add per block, the waves' partials in wave order."""
+    in fp32 as so many waves add it: blocks in groups of 256 values dealt out in
+    turn, one fused multiply-add per block, the waves' partials in wave order."""
     n = w.shape[0]
     s = oracle.isums(qtype, w, aq, m, n, k).astype(np.float64).reshape(m, n, -1, 2 if qtype == 1 else 1)
     blocks = w.reshape(n, -1, BLOCK[qtype][1])
@@ -58,10 +58,10 @@ def wave_sums(oracle, qtype, w, aq, m, k):
         x, y = rounded(0.125 * d * ad), s[..., 0]
         exact = 0.125 * d * ad * s[..., 0]
     group, total = 256 // BLOCK[qtype][0], None
-    for wave in range(16):
+    for wave in range(waves):
         acc = np.zeros((m, n))
         for b in range(blocks.shape[1]):
-            if b // group % 16 == wave:
+            if b // group % waves == wave:
                 acc = rounded(acc + x[..., b] * np.broadcast_to(y, s.shape[:3])[..., b])
         total = acc if total is None else rounded(total + acc)
     return exact.sum(-1), total
@@ -84,3 +84,22 @@ def test_automatic_path_as_exact_as_16_waves(hip, torch_gpu, oracle, qtype, m, n
     error = lambda x: np.sqrt(((x - exact) ** 2).mean() / (exact ** 2).mean())
     say(f"relative error {error(got):.3g}, 16 waves {error(waves):.3g}, path {hip.auto_path(qtype, m, n, k)}")
     assert error(got) <= 1.05 * error(waves)
+
+
+@pytest.mark.parametrize("qtype,m,n,k", [(1, 20, 9221, 1280), (1, 80, 9597, 2560), (1, 45, 20393, 1792),
+                                         (1, 33, 4096, 3328), (2, 20, 9222, 2304), (2, 128, 4096, 3328)])
+def test_tiles_at_other_k_as_exact_as_two_slices(hip, torch_gpu, oracle, qtype, m, n, k):
+    """At the k that PFNG_PATH_GEMV declines for m > 16 the 16-row tiles stand in
+    for GEMM tiles of at most two slices (about 30000 outputs: 1 % scatter)."""
+    torch = torch_gpu
+    say(f"rounding type={qtype} {m}x{n}x{k}")
+    w = random_weights(torch, qtype, n, k, seed=m + n + k)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    q = hip.quantize_activation(qtype, torch.randn((m, k), generator=g, device="cuda"))
+    cols = torch.randperm(n, generator=g, device="cuda")[:32768 // m]
+    exact, slices = wave_sums(oracle, qtype, w[cols].cpu().numpy(), q.cpu().numpy(), m, k, 2)
+    got = hip.mul_mat(qtype, w, q, m, n, k)[:, cols].double().cpu().numpy()
+    error = lambda x: np.sqrt(((x - exact) ** 2).mean() / (exact ** 2).mean())
+    say(f"relative error {error(got):.3g}, two slices {error(slices):.3g}")
+    assert error(got) <= 1.02 * error(slices)
