@@ -211,7 +211,7 @@ def test_half_split_copy_order(source, kernel, copies, after_half0, lead):
     check_half_split(_kernel_lines(asm, kernel), copies, after_half0, lead)
 
 
-def check_chunk_waits(lines: list[str], chunks: int, table_wait: int | None = None) -> None:
+def check_chunk_waits(lines: list[str], chunks: int, table_wait: int | None = None, reloads: bool = False) -> None:
     """The chunked MFMA tile GEMVs (from k = 4096, up to m = 128): no scratch memory
     (spill loads and stores would count in vmcnt and break the waits'
     arithmetic), and the vector-memory waits are exactly the designed ones: one
@@ -219,8 +219,20 @@ def check_chunk_waits(lines: list[str], chunks: int, table_wait: int | None = No
     everything. A kernel with a table wait (table_wait: its vmcnt) has it
     exactly once; it may be laid out after the loop body, so only its count is
     checked. (The iq2_xxs kernel has none: each wave's own table copy goes out
-    before its first weight copy, so the first vmcnt(3) covers it.)"""
-    assert not any(t.startswith("scratch_") or "buffer_store" in t for t in lines), "register spills"
+    before its first weight copy, so the first vmcnt(3) covers it.)
+    reloads: a register may be spilled across the rounds, its accesses ahead of
+    the round's first copy, and waited for there, or behind the last wait."""
+    spills = [i for i, t in enumerate(lines) if t.startswith("scratch_") or "buffer_store" in t]
+    if reloads:
+        first = next(i for i, t in enumerate(lines) if t.startswith("global_load_lds"))
+        ahead = [i for i in spills if i < first]
+        if ahead:
+            assert any(re.match(r"s_waitcnt .*vmcnt\(0\)", t) for t in lines[ahead[-1]:first]), "spills in flight at the copies"
+        waited = [i for i, t in enumerate(lines) if i > first and re.match(r"s_waitcnt .*vmcnt", t)][2 * chunks - 1]
+        assert not any(first < i < waited for i in spills), "register spills among the copies"
+        lines = lines[first:]
+    else:
+        assert not spills, "register spills"
     waits = [int(re.search(r"vmcnt\((\d+)\)", t).group(1)) for t in lines if re.match(r"s_waitcnt .*vmcnt", t)]
     if table_wait is not None:
         assert waits.count(table_wait) == 1, f"waits {waits}: expected one table wait vmcnt({table_wait})"
@@ -243,22 +255,33 @@ def test_chunk_wait_checker():
         check_chunk_waits(lines, 2, 8)
     with pytest.raises(AssertionError):  # two
         check_chunk_waits(["s_waitcnt vmcnt(8)"] + table, 2, 8)
+    reload = ["scratch_load_dword v0, off, off", "s_waitcnt vmcnt(0)"]
+    check_chunk_waits(reload + lines, 2, reloads=True)
+    with pytest.raises(AssertionError):  # still in flight when the copies start
+        check_chunk_waits(reload[:1] + lines, 2, reloads=True)
+    with pytest.raises(AssertionError):  # among the copies
+        check_chunk_waits(lines[:2] + reload[:1] + lines[2:], 2, reloads=True)
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
-@pytest.mark.parametrize("source,kernel,table_wait", [("gemv.hip", "gemv_q4_0_mfma_chunk_kernel", None),
-                                                      ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", None),
-                                                      ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", None)])
-@pytest.mark.parametrize("chunks", [1, 2, 3, 4, 8])
-@pytest.mark.parametrize("groups", [0, 16])
-def test_chunked_gemv_waits(source, kernel, table_wait, chunks, groups):
-    """Both forms: the group count read at run time (0, any number of rounds) and
-    fixed at 16 (k = 4096, one round)."""
+@pytest.mark.parametrize("source,kernel,form", [
+    ("gemv.hip", "gemv_q4_0_mfma_chunk_kernel", "Li0E"), ("gemv.hip", "gemv_q4_0_mfma_chunk_kernel", "Li16E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li16E"),
+    ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li0ELb0E"),
+    ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li16ELb0E"),
+    ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li0ELb1E")])
+@pytest.mark.parametrize("chunks", range(1, 9))
+def test_chunked_gemv_waits(source, kernel, form, chunks):
+    """Every form: the group count read at run time (0, any number of rounds; for
+    iq2_xxs also where rows do not share one alignment) and fixed at 16 (k = 4096,
+    one round). q4_K at seven chunks spills three lane addresses across its rounds."""
     out = os.path.join(PKG_DIR, "_build", source + ".s")
     subprocess.run(["make", "-s", "-C", PKG_DIR, out], check=True, capture_output=True, timeout=600)
     with open(out) as f:
         asm = f.read()
-    check_chunk_waits(_kernel_lines(asm, f"{kernel}ILi{chunks}ELi{groups}E"), chunks, table_wait)
+    check_chunk_waits(_kernel_lines(asm, f"{kernel}ILi{chunks}E{form}"), chunks,
+                      reloads=(kernel, form, chunks) == ("gemv_q4_K_mfma_chunk_kernel", "Li0E", 7))
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
