@@ -66,6 +66,7 @@ struct Q40Config {
     using Isums = Q40Config<BM, BN, WM, WN, KB, WK, AHEAD, 0, MINW>;  // of the diagnostic, which folds nothing
     static constexpr int kThreads = 64 * WM * WN * WK;
     static constexpr int kWaveBlocks = KB / WK;  // blocks per stage of one wave
+    static constexpr bool kTails = KB > 4;       // k % 128 == 0: stages of 4 blocks are always full
     static constexpr int TM = BM / WM / 32;  // 32x32 tiles per wave along m
     static constexpr int TN = BN / WN / 32;  // along n
     // staging pieces of 16 bytes: half an activation block, one weight block
@@ -140,7 +141,7 @@ __device__ __forceinline__ StageSlots stage_slots(int nb) {
     o.a = q4_0_act_piece(ra, pa, nb);
     const int rw = threadIdx.x / C::kWPerRow, jw = threadIdx.x % C::kWPerRow;
     o.w = q4_0_weight_piece(rw, jw, nb);
-    const int tail = nb % C::kKB;
+    const int tail = C::kTails ? nb % C::kKB : 0;
     o.a_past = tail && ja >= tail ? kPastEnd : 0u;
     o.w_past = tail && jw >= tail ? kPastEnd : 0u;
     o.sel_a = ja & 1 ? kOdd : kEven;

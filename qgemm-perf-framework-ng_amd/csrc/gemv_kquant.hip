@@ -1108,7 +1108,8 @@ __device__ __forceinline__ float sum_wave_partials(const float *p) {
 // The seven-chunk kernel with run-time strides holds its copies' lane addresses in
 // 128 VGPRs and spills three across the rounds, reloaded before a round's first
 // copy. Made to spill none (98 VGPRs, the addresses recomputed) it is slower: m =
-// 100, n = 4096 k = 2048 7.18 -> 7.42 us, 8192 20.3 -> 21.5, 11008 27.7 -> 29.1.
+// 100, n = 4096 k = 8192 20.3 -> 21.5 us, 11008 27.7 -> 29.1 (m = 112, 2048 7.18 ->
+// 7.42).
 template <int C, int kG>
 __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(const uint8_t *__restrict__ w,
                                                                              const uint8_t *__restrict__ a,

@@ -284,6 +284,33 @@ def test_chunked_gemv_waits(source, kernel, form, chunks):
                       reloads=(kernel, form, chunks) == ("gemv_q4_K_mfma_chunk_kernel", "Li0E", 7))
 
 
+def loop_bodies(lines: list[str]) -> list[list[str]]:
+    """The instructions between each label and a later branch back to it."""
+    at = {t[:-1]: i for i, t in enumerate(lines) if t.endswith(":")}
+    out = []
+    for i, t in enumerate(lines):
+        m = re.match(r"s_c?branch\S* (\S+)", t)
+        if m and at.get(m.group(1), i) < i:
+            out.append(lines[at[m.group(1)]:i])
+    return out
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
+def test_q4_0_gemm_loops_touch_no_scratch():
+    """No q4_0 GEMM tile reloads a spilled register inside its K loop: loads return
+    in order, so such a reload drains the staging pieces in flight."""
+    out = os.path.join(PKG_DIR, "_build", "gemm_mfma.hip.s")
+    subprocess.run(["make", "-s", "-C", PKG_DIR, out], check=True, capture_output=True, timeout=600)
+    with open(out) as f:
+        asm = f.read()
+    products = re.findall(r"^(\S*gemm_q4_0_kernel\S*EELb0E\S*):", asm, re.M)  # not the block sums
+    assert len(products) >= 8
+    for kernel in products:
+        loops = [b for b in loop_bodies(_kernel_lines(asm, kernel)) if any(t.startswith("v_mfma") for t in b)]
+        assert loops, f"{kernel}: no K loop found"
+        assert not any(t.startswith("scratch_") for b in loops for t in b), f"{kernel}: scratch in the K loop"
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
 @pytest.mark.parametrize("source", ["gemv.hip", "gemv_kquant.hip", "gemm_small.hip", "quantize.hip"])
 def test_kernel_arguments_preloaded(source):
