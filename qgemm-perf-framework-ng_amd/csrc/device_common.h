@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "load_offsets.h"
 #include "pfng_blocks.h"
 
 namespace pfng {
@@ -418,7 +419,7 @@ __device__ __forceinline__ void run_copy_exact(const uint8_t *src, uint32_t rstr
         const int col = col0 + p - r * kCols;
         if (r > rvalid - 1) r = rvalid - 1;
         uint32_t off = (uint32_t)r * rstride + 16u * (uint32_t)col;
-        if constexpr (kParity) off += 2u - 2u * (uint32_t)((first + r * odd) & 1);
+        if constexpr (kParity) off += 2u - (uint32_t)iq2_copy_odd(first + r * odd);
         __builtin_amdgcn_global_load_lds(src + off, (__attribute__((address_space(3))) void *)(dst + i * 1024), 16,
                                          0, 0);
     }
@@ -427,7 +428,7 @@ __device__ __forceinline__ void run_copy_exact(const uint8_t *src, uint32_t rstr
     const int col = col0 + p - r * kCols;
     if (r > rvalid - 1) r = rvalid - 1;
     uint32_t off = (uint32_t)r * rstride + 16u * (uint32_t)col + 4u * (uint32_t)(lane & 3);
-    if constexpr (kParity) off += 2u - 2u * (uint32_t)((first + r * odd) & 1);
+    if constexpr (kParity) off += 2u - (uint32_t)iq2_copy_odd(first + r * odd);
     __builtin_amdgcn_global_load_lds(src + off, (__attribute__((address_space(3))) void *)(dst + kFull * 1024), 4, 0,
                                      0);
 }

@@ -1126,7 +1126,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
     // at the block, on a dword, and H1 is the block's last 176 bytes (chunks
     // 8..18 would end 12 past it, for the last block past the rows).
     const bool even_rows = kG > 0 ? kG % 4 == 0 : nsb % 4 == 0;
-    const int h1s = even_rows ? 128 : 116;
+    const int h1s = even_rows ? kQ4kHalf1Chunk : kQ4kHalf1Block;
     constexpr int kH = run_copies<16, 11>();  // instructions per half (H1: 11 columns, H0: 9)
     static_assert(run_copies<16, 9>() == kH && run_copies<16, 9>() * 1024 <= 3072, "3 KB per run");
     static_assert(4 * C * 64 * 4 <= kChunkWaveBytes, "a wave's partials fit its buffers");
@@ -1338,11 +1338,11 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_iq2_xxs_mfma_chunk_kerne
             o2 = 2 * (wave & 7);
             run_copy_exact<16, 5>(w + ((size_t)n0 * nsb + sb) * kIq2Bytes - o2, nsb * kIq2Bytes, 0, n - n0, wl, cl);
         } else {
-            const int back = sb > 0 ? 12 : 0;
+            const int back = iq2_copy_back(sb);
             run_copy_exact<16, 5, true>(w + ((size_t)n0 * nsb + sb) * kIq2Bytes - back - 2, nsb * kIq2Bytes, 0, n - n0,
                                         wl, cl, nsb & 1, sb);  // n0 is even
             const int row = li < n - n0 ? li : n - n0 - 1;
-            o2 = back + 2 * ((sb + row * nsb) & 1);
+            o2 = back + iq2_copy_odd(sb + row * nsb);
         }
         copy_h0(0);
         copy_h1(0);

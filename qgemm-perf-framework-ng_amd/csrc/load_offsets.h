@@ -36,4 +36,17 @@ constexpr BufferOffset q4_0_stage_piece(uint32_t piece, uint32_t step, uint32_t 
     return {(piece + step) | past, stage};
 }
 
+// iq2_xxs weight blocks (66 bytes, at any even address) in the tile GEMV at every
+// k: their copies of 80 bytes start on a dword, 2 bytes before the block where its
+// index in the matrix is odd, and 12 more behind a row's first block, so that they
+// end at most 2 bytes past the block and only where the index is even.
+constexpr int iq2_copy_back(int super_block) { return super_block > 0 ? 12 : 0; }
+constexpr int iq2_copy_odd(int block) { return 2 * (block & 1); }
+
+// q8_K activation blocks (292 bytes) in the q4_K tile GEMV: byte at which the
+// second half's 176-byte copy starts, from the first half's start. Where rows
+// share one alignment that is 0..12 bytes before the block, and the halves are
+// 16-byte chunks; else it is the block, and the second half its last 176 bytes.
+constexpr int kQ4kHalf1Chunk = 128, kQ4kHalf1Block = 116;
+
 }  // namespace pfng

@@ -15,11 +15,16 @@ from test_gpu_exact import assert_bits_equal, dev, say
 
 pytestmark = pytest.mark.gpu
 
-# one, two, three and more stages of the 128x128 tiles; then a grid over which
-# the plan picks every tile, at k that fill the last stage of some and not of others
+# one, two, three and more stages of the 128x128 tiles; then a grid of m and n at k
+# that fill the last stage of some tiles and not of others. tests/test_plan.py checks
+# that the plan picks every tile here, with odd and even stage counts
 CASES = ([(2048, 4096, 128), (2000, 4100, 256), (1921, 4097, 384), (2048, 4096, 640)]
          + [(m, n, k) for m in (9, 33, 100, 200, 333, 700) for n in (100, 1500, 4100) for k in (128, 384, 1152, 2176)]
-         + [(40, 4100, 4096), (130, 4033, 4224), (500, 4000, 1664), (1000, 1500, 1280)])
+         + [(40, 4100, 4096), (130, 4033, 4224), (500, 4000, 1664), (1000, 1500, 1280)]
+         # 32x32 in 8 K-waves: one partial stage, two, three, three full; 32x64
+         + [(20, 100, 896), (20, 100, 1664), (37, 90, 2944), (20, 100, 3072), (20, 100, 1408), (500, 533, 896)]
+         # an even (128x128, 128x64, 64x64 in 2 K-waves) and an odd count (64x64)
+         + [(500, 10492, 256), (500, 2265, 1408), (500, 1832, 640), (500, 2265, 640)])
 
 
 # the tiles that fold their sums after every stage (128x64, 64x64 and its two K-waves), which the

@@ -19,13 +19,14 @@ def expected(oracle, qtype, x):
     return y.view(np.uint8).reshape(-1)
 
 
-@pytest.mark.parametrize("qtype,rows,k", [(0, 1, 32), (0, 63, 32), (0, 65, 32), (0, 255, 32), (0, 257, 96),
-                                          (1, 1, 256), (1, 7, 256), (1, 9, 256), (1, 31, 256), (1, 33, 768)])
-@pytest.mark.parametrize("offset", [0, 2])
+Q4_0_COUNTS = [(1, 32), (63, 32), (65, 32), (255, 32), (257, 96)]
+Q4_K_COUNTS = [(1, 256), (7, 256), (9, 256), (31, 256), (33, 768)]  # outputs 16-byte aligned
+
+
+@pytest.mark.parametrize("qtype,rows,k,offset", [(0, *c, o) for c in Q4_0_COUNTS for o in (0, 2)]
+                         + [(1, *c, 0) for c in Q4_K_COUNTS])
 def test_block_counts(hip, torch_gpu, oracle, qtype, rows, k, offset):
     torch = torch_gpu
-    if qtype == 1 and offset:
-        pytest.skip("q4_K outputs are 16-byte aligned")
     say(f"weight quantizer type={qtype} rows={rows} k={k} offset={offset}")
     x = np.random.default_rng(rows + k).standard_normal((rows, k)).astype(np.float32)
     expect = expected(oracle, qtype, x)
@@ -105,17 +106,43 @@ def test_q4_0_infinite_and_nan(hip, torch_gpu, oracle):
 
 
 def test_q4_K_infinite_and_nan(hip, torch_gpu, oracle):
-    """A super-block with an infinite value (its range, and so every quotient,
-    leaves the correction steps' bounds) or a NaN beside finite values."""
+    """Super-blocks with infinities and NaN, each case in a wave (eight
+    super-blocks) of its own, whole super-blocks byte for byte: an infinite value
+    makes its sub-block's range infinite, which takes the wave out of the
+    correction steps' bounds; a NaN leaves the range finite, so it reaches the
+    correction steps (unless all of its sub-block is NaN) and quantizes to 0.
+    The reference passes over a NaN that is not its sub-block's first value."""
     torch = torch_gpu
-    say("q4_K inf / nan")
-    x = np.random.default_rng(3).standard_normal((4, 512)).astype(np.float32)
-    x[0, 40] = np.inf
-    x[1, 300] = -np.inf
-    x[2, 33] = np.nan
-    got = hip.quantize_weights_gpu(1, dev(torch, x)).cpu().numpy()
-    expect = expected(oracle, 1, x).reshape(4, -1)
-    # the packed scales of a super-block whose scale is infinite or NaN come
-    # from float -> int conversions of NaN; compare the finite super-blocks
-    for r, b in [(0, 1), (1, 0), (3, 0), (3, 1), (2, 1)]:
-        assert np.array_equal(got[r, 144 * b:144 * b + 144], expect[r, 144 * b:144 * b + 144]), (r, b)
+    nan, inf = np.float32(np.nan), np.float32(np.inf)
+    plain = np.random.default_rng(3).standard_normal((8, 256)).astype(np.float32)
+    places = {"+inf": [(0, 40, inf)], "-inf": [(1, 77, -inf)], "both": [(2, 3, inf), (2, 9, -inf), (5, 200, inf)],
+              "NaN": [(0, 33, nan), (3, 1, nan), (3, 255, nan), (6, 130, -nan)],
+              "all but one NaN": [(4, i, nan) for i in range(33, 64)],
+              "a NaN sub-block": [(4, i, nan) for i in range(32, 64)],
+              "NaN beside inf": [(7, 65, nan), (7, 70, inf)]}
+    for name, values in places.items():
+        x = plain.copy()
+        for b, i, v in values:
+            x[b, i] = v
+        say(f"q4_K inf / nan: {name}")
+        got = hip.quantize_weights_gpu(1, dev(torch, x)).cpu().numpy().reshape(8, 144)
+        bad = np.flatnonzero((got != expected(oracle, 1, x).reshape(8, 144)).any(1))
+        assert bad.size == 0, f"{name}: super-blocks {bad} differ"
+
+
+def test_q4_K_leading_nan(hip, torch_gpu, oracle):
+    """A NaN that is its sub-block's first value makes the reference's range NaN
+    (its minimum starts there); the kernel's minimum and maximum pass over it like
+    any other, so the bytes are those of the same values with the NaN second."""
+    torch = torch_gpu
+    say("q4_K leading nan")
+    x = np.random.default_rng(4).standard_normal((8, 256)).astype(np.float32)
+    x[2, 64] = np.nan
+    moved = x.copy()
+    moved[2, [64, 65]] = x[2, [65, 64]]
+    got = hip.quantize_weights_gpu(1, dev(torch, x)).cpu().numpy().reshape(8, 144)
+    expect = expected(oracle, 1, moved).reshape(8, 144).copy()
+    # sub-block 2: the low nibbles of qs[32..63], whose first two values change places back
+    q = expect[2, 16 + 32:16 + 34]
+    expect[2, 16 + 32:16 + 34] = (q & 0xF0) | (q[::-1] & 0x0F)
+    assert np.array_equal(got, expect)
