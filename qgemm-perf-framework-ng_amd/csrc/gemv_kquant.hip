@@ -1089,8 +1089,8 @@ __host__ __device__ constexpr int q4k_chunk_lds_bytes(int c) {
 // order (k = 4096) or the GEMM tiles' slices (k = 2816): q4_K 1.03e-7 -> 8.7e-8 and
 // 9.1e-8 -> 8.5e-8, iq2_xxs 8.4e-8 -> 6.5e-8 and 6.0e-8 -> 6.3e-8 in fp32; in fp64
 // 7.2e-8, 7.2e-8, 4.3e-8 and 4.3e-8, for 1-2 % of the time at n = 4096 (4096 x 4096,
-// m = 128 q4_K 15.35 -> 15.49 us) and up to 8 % on wide outputs (45x20393x1792 17.7
-// -> 19.1). So fp64 is for the rows that GEMM slices would add more exactly than
+// m = 128 q4_K 15.35 -> 15.49 us) and up to 5 % on wide outputs (45x20393x1792 17.7
+// -> 18.5). So fp64 is for the rows that GEMM slices would add more exactly than
 // fp32 pairs: iq2_xxs at every such k, q4_K up to 14 super-blocks from m = 17
 // (20x9221x1280 8.5e-8 -> 7.7e-8, two slices 8.0e-8).
 template <int kStride, class T = float, int kN = kKqMfWaves>
@@ -1110,7 +1110,11 @@ __device__ __forceinline__ float sum_wave_partials(const float *p) {
 // copy. Made to spill none (98 VGPRs, the addresses recomputed) it is slower: m =
 // 100, n = 4096 k = 8192 20.3 -> 21.5 us, 11008 27.7 -> 29.1 (m = 112, 2048 7.18 ->
 // 7.42).
-template <int C, int kG>
+// kFew: rows of at most 14 super-blocks, no multiple of four of them, whose partials
+// are added in fp64. A form of its own: as a branch at run time the fp64 code cost
+// the other rows up to 4 % and these as much (45x2048x2048 4.54 -> 4.69 us, 48x6144x2048
+// 7.70 -> 8.01; 20x9221x1280 8.15 -> 8.52, 45x4096x1792 4.66 -> 4.78).
+template <int C, int kG, bool kFew = false>
 __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(const uint8_t *__restrict__ w,
                                                                              const uint8_t *__restrict__ a,
                                                                              float *__restrict__ c, int m, int n,
@@ -1125,7 +1129,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
     // the copies to 16-byte boundaries (H1 = chunks 8..18); otherwise they start
     // at the block, on a dword, and H1 is the block's last 176 bytes (chunks
     // 8..18 would end 12 past it, for the last block past the rows).
-    const bool even_rows = kG > 0 ? kG % 4 == 0 : nsb % 4 == 0;
+    const bool even_rows = !kFew && (kG > 0 ? kG % 4 == 0 : nsb % 4 == 0);
     const int h1s = even_rows ? kQ4kHalf1Chunk : kQ4kHalf1Block;
     constexpr int kH = run_copies<16, 11>();  // instructions per half (H1: 11 columns, H0: 9)
     static_assert(run_copies<16, 9>() == kH && run_copies<16, 9>() * 1024 <= 3072, "3 KB per run");
@@ -1239,12 +1243,10 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[wave * kStride + (ch * 4 + r) * 64 + lane] = acc[ch][r];
     __syncthreads();
-    // (one chunk: m <= 16)
-    const bool few = C > 1 && kG == 0 && !even_rows && nsb <= 14;
     const int col = n0 + li;
     for (int g = wave; g < 4 * C; g += kKqMfWaves) {
         const float *p = red + g * 64 + lane;
-        const float s = few ? sum_wave_partials<kStride, double, 14>(p) : sum_wave_partials<kStride>(p);
+        const float s = kFew ? sum_wave_partials<kStride, double, 14>(p) : sum_wave_partials<kStride>(p);
         const int row = 16 * (g / 4) + 4 * q + g % 4;
         if (col < n && row < m) store_through(&c[(size_t)row * n + col], s);
     }
@@ -1433,6 +1435,8 @@ void launch_kq_chunk(bool q4k, const uint8_t *w, const uint8_t *a, float *c, int
     const size_t lds = q4k ? (size_t)q4k_chunk_lds_bytes(C) : (size_t)iq2_chunk_lds_bytes(C);
     if (q4k && nsb == kKqMfWaves)
         hipLaunchKernelGGL((gemv_q4_K_mfma_chunk_kernel<C, kKqMfWaves>), grid, block, lds, stream, w, a, c, m, n, nsb);
+    else if (q4k && C > 1 && nsb % 4 && nsb <= 14)
+        hipLaunchKernelGGL((gemv_q4_K_mfma_chunk_kernel<C, 0, (C > 1)>), grid, block, lds, stream, w, a, c, m, n, nsb);
     else if (q4k)
         hipLaunchKernelGGL((gemv_q4_K_mfma_chunk_kernel<C, 0>), grid, block, lds, stream, w, a, c, m, n, nsb);
     else if (nsb == kKqMfWaves)

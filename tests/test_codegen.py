@@ -264,24 +264,40 @@ def test_chunk_wait_checker():
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
-@pytest.mark.parametrize("source,kernel,form", [
+@pytest.mark.parametrize("source,kernel,form,chunks", [(*f, c) for f in [
     ("gemv.hip", "gemv_q4_0_mfma_chunk_kernel", "Li0E"), ("gemv.hip", "gemv_q4_0_mfma_chunk_kernel", "Li16E"),
-    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0E"),
-    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li16E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0ELb0E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li16ELb0E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0ELb1E"),
     ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li0ELb0E"),
     ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li16ELb0E"),
-    ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li0ELb1E")])
-@pytest.mark.parametrize("chunks", range(1, 9))
+    ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li0ELb1E")]
+    for c in range(1, 9) if (*f[1:], c) != ("gemv_q4_K_mfma_chunk_kernel", "Li0ELb1E", 1)])
 def test_chunked_gemv_waits(source, kernel, form, chunks):
     """Every form: the group count read at run time (0, any number of rounds; for
-    iq2_xxs also where rows do not share one alignment) and fixed at 16 (k = 4096,
-    one round). q4_K at seven chunks spills three lane addresses across its rounds."""
+    iq2_xxs also where rows do not share one alignment, for q4_K also with the fp64
+    sum of short rows, from two chunks) and fixed at 16 (k = 4096, one round). q4_K at
+    seven chunks spills three lane addresses across its rounds."""
     out = os.path.join(PKG_DIR, "_build", source + ".s")
     subprocess.run(["make", "-s", "-C", PKG_DIR, out], check=True, capture_output=True, timeout=600)
     with open(out) as f:
         asm = f.read()
     check_chunk_waits(_kernel_lines(asm, f"{kernel}ILi{chunks}E{form}"), chunks,
-                      reloads=(kernel, form, chunks) == ("gemv_q4_K_mfma_chunk_kernel", "Li0E", 7))
+                      reloads=(kernel, form[:3], chunks) == ("gemv_q4_K_mfma_chunk_kernel", "Li0", 7))
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
+@pytest.mark.parametrize("chunks", range(2, 9))
+def test_q4_K_gemv_fp64_sums_in_their_own_form(chunks):
+    """The fp64 sum of short rows is no branch of the kernel that all other rows
+    run (as one it cost them up to 4 %)."""
+    out = os.path.join(PKG_DIR, "_build", "gemv_kquant.hip.s")
+    subprocess.run(["make", "-s", "-C", PKG_DIR, out], check=True, capture_output=True, timeout=600)
+    with open(out) as f:
+        asm = f.read()
+    for form, fp64 in (("Li0ELb0E", False), ("Li16ELb0E", False), ("Li0ELb1E", True)):
+        lines = _kernel_lines(asm, f"gemv_q4_K_mfma_chunk_kernelILi{chunks}E{form}")
+        assert any(t.startswith("v_add_f64") for t in lines) == fp64, form
 
 
 def loop_bodies(lines: list[str]) -> list[list[str]]:
