@@ -69,6 +69,12 @@ struct Q40Config {
     static constexpr bool kTails = KB > 4;       // k % 128 == 0: stages of 4 blocks are always full
     static constexpr int TM = BM / WM / 32;  // 32x32 tiles per wave along m
     static constexpr int TN = BN / WN / 32;  // along n
+    // whether the last two stages run behind the K loop too, without its loads of
+    // further stages, which the last stage of an even number would wait for (the
+    // copies of two larger stages cost the 128x128 tile 200 bytes of spills). us in
+    // the loop and apart, q4_0 100x400x512 4.97 / 4.42, 512x4096x2048 16.7 / 15.9,
+    // 64x16640x1024 10.5 / 9.9; long or odd rows within 1 %.
+    static constexpr bool kLastApart = TM * TN == 1;
     // staging pieces of 16 bytes: half an activation block, one weight block
     static constexpr int kActPerRow = 2 * KB, kWPerRow = KB;
     static constexpr int kActPT = BM * kActPerRow / kThreads;  // pieces per thread
@@ -400,8 +406,8 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
     // once with the piece kAhead pieces on (so kAhead pieces are in flight).
     // Past the end the stage index is clamped, so the loop body has no
     // divergent control flow; rounds of two stages make register set and
-    // buffer compile-time constants, and an odd last stage is computed after
-    // the loop.
+    // buffer compile-time constants, and an odd last stage (kLastApart: the last
+    // one or two) is computed after the loop.
     const int stages = (nb + C::kKB - 1) / C::kKB;
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(a + (size_t)m0 * nb * 34), 0,
@@ -431,8 +437,9 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
     __syncthreads();
     const int tb = wk * C::kWaveBlocks;
     int s = 0;
-    // one stage of a round (R = 0 or 1), from buffer R
-    auto stage = [&](auto R) __attribute__((always_inline)) {
+    // one stage of a round (R = 0 or 1), from buffer R; More: the pieces of stages
+    // after the next are loaded
+    auto stage = [&](auto R, auto More) __attribute__((always_inline)) {
         constexpr int rr = decltype(R)::value;
         __builtin_amdgcn_sched_barrier(0);
         compute_stage<C, kIsums, C::kFold == 1 || (C::kFold == 2 && rr == 0)>(
@@ -441,21 +448,34 @@ __global__ __launch_bounds__(C::kThreads, C::kMinWavesPerEU) void gemm_q4_0_kern
                 PieceRegs &r = regs[(rr * C::kPieces + p) % C::kAhead];
                 store_piece<C>(lds + (rr ^ 1) * C::kBufBytes, slots, p, r);
                 const int x = p + C::kAhead;
-                load(s + rr + 1 + x / C::kPieces, x % C::kPieces, r);
+                if (decltype(More)::value || x < C::kPieces) load(s + rr + 1 + x / C::kPieces, x % C::kPieces, r);
             });
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
     };
-    for (; s + 1 < stages; s += 2) {
-        stage(std::integral_constant<int, 0>{});
+    // the last stage, from buffer R
+    auto last_stage = [&](auto R) __attribute__((always_inline)) {
+        constexpr int rr = decltype(R)::value;
+        compute_stage<C, kIsums, C::kFold == 1 || (C::kFold == 2 && rr == 0)>(
+            lds, rr, acc, isums, m, n, nb, m0, n0, s + rr, tb, lane, wave_m, wave_n, [](int) {});
+        fold();
+    };
+    using First = std::integral_constant<int, 0>;
+    using Second = std::integral_constant<int, 1>;
+    for (; s + 1 + C::kLastApart < stages; s += 2) {
+        stage(First{}, std::true_type{});
         if constexpr (C::kFold == 1) fold();
-        stage(std::integral_constant<int, 1>{});
+        stage(Second{}, std::true_type{});
         fold();
     }
-    if (s < stages) {
-        compute_stage<C, kIsums, (C::kFold > 0)>(lds, 0, acc, isums, m, n, nb, m0, n0, s, tb, lane, wave_m, wave_n,
-                                           [](int) {});
-        fold();
+    if (!C::kLastApart) {
+        if (s < stages) last_stage(First{});
+    } else if (s + 1 < stages) {
+        stage(First{}, std::false_type{});
+        if constexpr (C::kFold == 1) fold();
+        last_stage(Second{});
+    } else {
+        last_stage(First{});
     }
     if constexpr (C::kFold > 0 && !kIsums) {
 #pragma unroll

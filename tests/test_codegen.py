@@ -328,6 +328,30 @@ def test_q4_0_gemm_loops_touch_no_scratch():
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
+def test_q4_0_gemm_last_stages_load_nothing():
+    """The tiles with one 32x32 tile per wave run the last one or two stages behind
+    the K loop, without the loop's loads of further stages (clamped to the last
+    one there): the last of an even number of stages would wait for them."""
+    out = os.path.join(PKG_DIR, "_build", "gemm_mfma.hip.s")
+    subprocess.run(["make", "-s", "-C", PKG_DIR, out], check=True, capture_output=True, timeout=600)
+    with open(out) as f:
+        asm = f.read()
+    seen = 0
+    for kernel in re.findall(r"^(\S*gemm_q4_0_kernel\S*EELb0E\S*):", asm, re.M):
+        bm, bn, wm, wn, kb, wk = (int(x) for x in re.findall(r"Li(\d+)E", kernel)[:6])
+        if (bm // wm, bn // wn) != (32, 32):
+            continue
+        seen += 1
+        lines = _kernel_lines(asm, kernel)
+        loop = next(b for b in loop_bodies(lines) if any(t.startswith("v_mfma_i32") for t in b))
+        at = next(i for i in range(len(lines)) if lines[i:i + len(loop)] == loop)
+        behind = lines[at + len(loop):]
+        assert sum(t.startswith("v_mfma_i32") for t in behind) == 3 * (kb // wk), kernel
+        assert not any(t.startswith("buffer_load") for t in behind), kernel
+    assert seen >= 7
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
 @pytest.mark.parametrize("source", ["gemv.hip", "gemv_kquant.hip", "gemm_small.hip", "quantize.hip"])
 def test_kernel_arguments_preloaded(source):
     """Every kernel asks for its first kernel-argument dwords in SGPRs at wave
