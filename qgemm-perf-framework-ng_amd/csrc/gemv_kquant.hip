@@ -1110,11 +1110,16 @@ __device__ __forceinline__ float sum_wave_partials(const float *p) {
 // copy. Made to spill none (98 VGPRs, the addresses recomputed) it is slower: m =
 // 100, n = 4096 k = 8192 20.3 -> 21.5 us, 11008 27.7 -> 29.1 (m = 112, 2048 7.18 ->
 // 7.42).
-// kFew: rows of at most 14 super-blocks, no multiple of four of them, whose partials
-// are added in fp64. A form of its own: as a branch at run time the fp64 code cost
-// the other rows up to 4 % and these as much (45x2048x2048 4.54 -> 4.69 us, 48x6144x2048
-// 7.70 -> 8.01; 20x9221x1280 8.15 -> 8.52, 45x4096x1792 4.66 -> 4.78).
-template <int C, int kG, bool kFew = false>
+// Forms of the q4_K kernel. kAny: any nsb, told apart at run time. kAligned: nsb % 4
+// == 0, at the fixed nsb of k = 4096 and for two and three chunks (us against kAny:
+// 20x1058x5120 4.89 / 5.08, 20x4096x8192 7.69 / 7.84, 45x6144x2048 7.77 / 7.97; one and
+// four to six chunks within 1 %, seven slower: 112x4096x8192 21.9 / 20.8). kFew: nsb <=
+// 14 and nsb % 4 != 0 from two chunks, the partials added in fp64; as a branch at run
+// time that code cost the other rows up to 4 % and these as much (45x2048x2048 4.54 ->
+// 4.69, 48x6144x2048 7.70 -> 8.01; 20x9221x1280 8.15 -> 8.52, 45x4096x1792 4.66 -> 4.78).
+enum class Q4kRows { kAligned, kAny, kFew };
+
+template <int C, int kG, Q4kRows R>
 __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(const uint8_t *__restrict__ w,
                                                                              const uint8_t *__restrict__ a,
                                                                              float *__restrict__ c, int m, int n,
@@ -1129,7 +1134,8 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
     // the copies to 16-byte boundaries (H1 = chunks 8..18); otherwise they start
     // at the block, on a dword, and H1 is the block's last 176 bytes (chunks
     // 8..18 would end 12 past it, for the last block past the rows).
-    const bool even_rows = !kFew && (kG > 0 ? kG % 4 == 0 : nsb % 4 == 0);
+    static_assert(kG == 0 || (kG % 4 == 0 && R == Q4kRows::kAligned), "the fixed form has aligned rows");
+    const bool even_rows = R == Q4kRows::kAligned || (R == Q4kRows::kAny && nsb % 4 == 0);
     const int h1s = even_rows ? kQ4kHalf1Chunk : kQ4kHalf1Block;
     constexpr int kH = run_copies<16, 11>();  // instructions per half (H1: 11 columns, H0: 9)
     static_assert(run_copies<16, 9>() == kH && run_copies<16, 9>() * 1024 <= 3072, "3 KB per run");
@@ -1246,7 +1252,7 @@ __global__ __launch_bounds__(kKqMfWaves * 64) void gemv_q4_K_mfma_chunk_kernel(c
     const int col = n0 + li;
     for (int g = wave; g < 4 * C; g += kKqMfWaves) {
         const float *p = red + g * 64 + lane;
-        const float s = kFew ? sum_wave_partials<kStride, double, 14>(p) : sum_wave_partials<kStride>(p);
+        const float s = R == Q4kRows::kFew ? sum_wave_partials<kStride, double, 14>(p) : sum_wave_partials<kStride>(p);
         const int row = 16 * (g / 4) + 4 * q + g % 4;
         if (col < n && row < m) store_through(&c[(size_t)row * n + col], s);
     }
@@ -1433,12 +1439,17 @@ void launch_kq_chunk(bool q4k, const uint8_t *w, const uint8_t *a, float *c, int
                      hipStream_t stream) {
     const dim3 grid((unsigned)((n + 15) / 16)), block(kKqMfWaves * 64);
     const size_t lds = q4k ? (size_t)q4k_chunk_lds_bytes(C) : (size_t)iq2_chunk_lds_bytes(C);
+    constexpr Q4kRows kAlignedRows = C == 2 || C == 3 ? Q4kRows::kAligned : Q4kRows::kAny;
+    constexpr Q4kRows kFewRows = C > 1 ? Q4kRows::kFew : Q4kRows::kAny;
+    auto q4_K = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, lds, stream, w, a, c, m, n, nsb); };
     if (q4k && nsb == kKqMfWaves)
-        hipLaunchKernelGGL((gemv_q4_K_mfma_chunk_kernel<C, kKqMfWaves>), grid, block, lds, stream, w, a, c, m, n, nsb);
-    else if (q4k && C > 1 && nsb % 4 && nsb <= 14)
-        hipLaunchKernelGGL((gemv_q4_K_mfma_chunk_kernel<C, 0, (C > 1)>), grid, block, lds, stream, w, a, c, m, n, nsb);
+        q4_K(gemv_q4_K_mfma_chunk_kernel<C, kKqMfWaves, Q4kRows::kAligned>);
+    else if (q4k && nsb % 4 == 0)
+        q4_K(gemv_q4_K_mfma_chunk_kernel<C, 0, kAlignedRows>);
+    else if (q4k && nsb <= 14)
+        q4_K(gemv_q4_K_mfma_chunk_kernel<C, 0, kFewRows>);
     else if (q4k)
-        hipLaunchKernelGGL((gemv_q4_K_mfma_chunk_kernel<C, 0>), grid, block, lds, stream, w, a, c, m, n, nsb);
+        q4_K(gemv_q4_K_mfma_chunk_kernel<C, 0, Q4kRows::kAny>);
     else if (nsb == kKqMfWaves)
         hipLaunchKernelGGL((gemv_iq2_xxs_mfma_chunk_kernel<C, kKqMfWaves>), grid, block, lds, stream, w, a, c, m, n,
                            nsb);

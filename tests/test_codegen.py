@@ -266,18 +266,20 @@ def test_chunk_wait_checker():
 @pytest.mark.skipif(not os.path.exists(HIPCC) or shutil.which("make") is None, reason="needs hipcc and make")
 @pytest.mark.parametrize("source,kernel,form,chunks", [(*f, c) for f in [
     ("gemv.hip", "gemv_q4_0_mfma_chunk_kernel", "Li0E"), ("gemv.hip", "gemv_q4_0_mfma_chunk_kernel", "Li16E"),
-    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0ELb0E"),
-    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li16ELb0E"),
-    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0ELb1E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li16ELNS0_7Q4kRowsE0E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0ELNS0_7Q4kRowsE0E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0ELNS0_7Q4kRowsE1E"),
+    ("gemv_kquant.hip", "gemv_q4_K_mfma_chunk_kernel", "Li0ELNS0_7Q4kRowsE2E"),
     ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li0ELb0E"),
     ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li16ELb0E"),
     ("gemv_kquant.hip", "gemv_iq2_xxs_mfma_chunk_kernel", "Li0ELb1E")]
-    for c in range(1, 9) if (*f[1:], c) != ("gemv_q4_K_mfma_chunk_kernel", "Li0ELb1E", 1)])
+    for c in {"Li0ELNS0_7Q4kRowsE0E": (2, 3), "Li0ELNS0_7Q4kRowsE2E": range(2, 9)}.get(f[2], range(1, 9))])
 def test_chunked_gemv_waits(source, kernel, form, chunks):
     """Every form: the group count read at run time (0, any number of rounds; for
-    iq2_xxs also where rows do not share one alignment, for q4_K also with the fp64
-    sum of short rows, from two chunks) and fixed at 16 (k = 4096, one round). q4_K at
-    seven chunks spills three lane addresses across its rounds."""
+    iq2_xxs also where rows do not share one alignment; q4_K's forms: aligned rows at
+    two and three chunks, any, and short rows with an fp64 sum from two) and fixed at 16
+    (k = 4096, one round). q4_K at seven chunks spills three lane addresses across its
+    rounds."""
     out = os.path.join(PKG_DIR, "_build", source + ".s")
     subprocess.run(["make", "-s", "-C", PKG_DIR, out], check=True, capture_output=True, timeout=600)
     with open(out) as f:
@@ -295,7 +297,10 @@ def test_q4_K_gemv_fp64_sums_in_their_own_form(chunks):
     subprocess.run(["make", "-s", "-C", PKG_DIR, out], check=True, capture_output=True, timeout=600)
     with open(out) as f:
         asm = f.read()
-    for form, fp64 in (("Li0ELb0E", False), ("Li16ELb0E", False), ("Li0ELb1E", True)):
+    forms = [("Li16ELNS0_7Q4kRowsE0E", False), ("Li0ELNS0_7Q4kRowsE1E", False), ("Li0ELNS0_7Q4kRowsE2E", True)]
+    if chunks in (2, 3):
+        forms.append(("Li0ELNS0_7Q4kRowsE0E", False))
+    for form, fp64 in forms:
         lines = _kernel_lines(asm, f"gemv_q4_K_mfma_chunk_kernelILi{chunks}E{form}")
         assert any(t.startswith("v_add_f64") for t in lines) == fp64, form
 
