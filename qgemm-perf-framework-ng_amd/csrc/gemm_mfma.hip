@@ -640,7 +640,11 @@ int64_t q4_0_tile_ns(int config, int64_t m, int64_t n, int64_t k, int cus) {
     }
     case kCfgSmall4: {
         const int64_t r = rounds(64, 64), rest = r % 4;
-        return r / 4 * (2200 + 125 * k / 10) + (rest ? 1800 + (rest > 1 ? 105 : 83) * k / 10 : 0);
+        // short rows beyond four rounds wait for the outputs of the rounds before: us
+        // here and on the 128x128 tile 1335x4488x128 10.8 / 9.3, 1531x7108x512 30.0 /
+        // 27.9, 2048x14336x128 31.6 / 27.9 (1945x4367x640 29.2 / 31.4 stays)
+        const int64_t late = r > 4 && k <= 1024 ? 800 + (rest ? 400 : 0) : 0;
+        return late + r / 4 * (2200 + 125 * k / 10) + (rest ? 1800 + (rest > 1 ? 105 : 83) * k / 10 : 0);
     }
     case kCfgWideK4: return rounds(32, 64) * (1800 + 22 * padded(512) / 10);
     case kCfgTiny: {

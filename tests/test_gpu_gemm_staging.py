@@ -24,7 +24,9 @@ CASES = ([(2048, 4096, 128), (2000, 4100, 256), (1921, 4097, 384), (2048, 4096, 
          # 32x32 in 8 K-waves: one partial stage, two, three, three full; 32x64
          + [(20, 100, 896), (20, 100, 1664), (37, 90, 2944), (20, 100, 3072), (20, 100, 1408), (500, 533, 896)]
          # an even (128x128, 128x64, 64x64 in 2 K-waves) and an odd count (64x64)
-         + [(500, 10492, 256), (500, 2265, 1408), (500, 1832, 640), (500, 2265, 640)])
+         + [(500, 10492, 256), (500, 2265, 1408), (500, 1832, 640), (500, 2265, 640)]
+         # an even count (64x64 in 2 waves)
+         + [(900, 4100, 512)])
 
 
 # the tiles that fold their sums after every stage (128x64, 64x64 and its two K-waves), which the
