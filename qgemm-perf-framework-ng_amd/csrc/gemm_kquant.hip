@@ -779,18 +779,26 @@ hipError_t dispatch(const void *w, const void *a, float *c, const MfmaPlan &plan
 int64_t kq_tile_ns(bool q4k, int config, int64_t m, int64_t n, int64_t k, int cus) {
     auto rounds = [&](int64_t bm, int64_t bn) { return (tiles_of(m, n, bm, bn) + cus - 1) / cus; };
     const int64_t r64 = rounds(64, 64), r128 = rounds(128, 64), r32 = rounds(32, 32);
+    // q4_K: an odd number of super-blocks takes two slices as long as one more (300x300,
+    // us at k = 256, 512, 768, 1024: two slices 5.0, 5.0, 6.1, 6.0, four 5.8, 5.7, 5.9, 5.9).
+    // Longer rows hide that in the other workgroup of a CU (32 x 32) and in the taller
+    // tile's work (128 x 64). With k as it is 46x4161x256 ran in 5.3 us (32 x 32 4.8),
+    // 17x20060x256 in 8.6 (128 x 64 6.0), 281x12579x1280 in 38.5 (128 x 64 with one slice
+    // 31.3). From the fifth round on a round of 32 x 32 tiles costs a fifth more
+    // (142x17524x1280 35.5, 29.3 on the 128 x 64 tile; 141x16729x1792 42.7, 41.3).
+    const int64_t k2 = q4k ? (k + 511) / 512 * 512 : k, k2s = k < 1024 ? k2 : k, k4 = q4k && k <= 1024 ? 900 : k;
     switch (config) {
     case kCfgBig:
         return q4k ? r128 / 2 * (2600 + 135 * k / 10) + r128 % 2 * (1900 + 82 * k / 10)
                    : r128 / 2 * (2300 + 116 * k / 10) + r128 % 2 * (2000 + 69 * k / 10);
-    case kCfgBigS2: return r128 * (q4k ? 2400 + 69 * k / 10 : 2600 + 56 * k / 10);
-    case kCfgSmallS2: return r64 * (q4k ? 1300 + 48 * k / 10 : 1500 + 425 * k / 100);
+    case kCfgBigS2: return r128 * (q4k ? 2400 + 69 * k2s / 10 : 2600 + 56 * k / 10);
+    case kCfgSmallS2: return r64 * (q4k ? 1300 + 48 * k2 / 10 : 1500 + 425 * k / 100);
     case kCfgMid2:
     case kCfgMid2D:
         return (config == kCfgMid2D ? 350 : 0) +
-               (q4k ? 1000 + 26 * k / 10 + (r32 - 1) * (400 + 16 * k / 10)
+               (q4k ? 1000 + 26 * k2s / 10 + (r32 > 4 ? 6 * r32 - 9 : 5 * r32 - 5) * (400 + 16 * k2s / 10) / 5
                     : r32 / 2 * (800 + 39 * k / 10) + r32 % 2 * (1500 + 315 * k / 100));
-    default: return r32 * (1500 + (q4k ? 22 : 25) * k / 10);
+    default: return r32 * (1500 + (q4k ? 22 : 25) * k4 / 10);
     }
 }
 

@@ -1,4 +1,4 @@
-"""The q4_0 GEMM plan (csrc/gemm_mfma.hip, on the CPU): the staging tests reach
+"""The GEMM plans (csrc/gemm_mfma.hip and gemm_kquant.hip, on the CPU): the staging tests reach
 every tile, and the automatic path's tiles keep to their rounding limit over
 many shapes."""
 from __future__ import annotations
@@ -103,3 +103,16 @@ def test_automatic_tiles_round_no_more_than_the_gemv(pkg, plan):
                 moved.add(config)
                 assert tile_rounding(config, k // 32) <= 1.03 * limit, (m, n, k, config)
     assert {2, 4, 8} & moved and {1, 3} & moved  # both ways of folding
+
+
+@pytest.mark.parametrize("qtype,m,n,k,config", [
+    (0, 1335, 4488, 128, 0), (0, 1531, 7108, 512, 0), (0, 2048, 14336, 128, 0), (0, 1945, 4367, 640, 10),
+    (1, 46, 4161, 256, 3), (1, 17, 20060, 256, 0), (1, 281, 12579, 1280, 0), (1, 142, 17524, 1280, 0),
+    (1, 300, 300, 512, 3), (1, 300, 300, 1024, 5)])
+def test_plan_takes_the_measured_tile(pkg, qtype, m, n, k, config):
+    """Shapes on which the tiles differ by 2 to 45 %, the predicted times by little:
+    the plan is the tile measured fastest among those as exact."""
+    f = pkg.lib()._ZN4pfng9plan_mfmaEilllib
+    f.restype = Plan
+    f.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_bool]
+    assert f(qtype, m, n, k, CUS, True).config == config
