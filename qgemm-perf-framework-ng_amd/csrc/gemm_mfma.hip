@@ -18,16 +18,15 @@
 // write port, so an item's two MFMAs (64 cycles) and its 32 VALU operations
 // (2 cycles each: a subtraction that turns S16 into fp32, see based_sum, and
 // the FMA) add up instead of overlapping. Measured in a 128x128-tile workgroup pair per
-// CU at 2.0 GHz: 163 cycles an item, 126 with the staging left out. Before the
-// staging was cut into pieces it was a phase of its own after each stage, with
-// one block pair (68 / 36 bytes) per thread and load, so that a load touched 32
-// rows; together with the conversion v_cvt_f32_i32 (about 5 cycles) us then and
-// now, in one process: 2048x11008x4096 267.9 -> 246.3 (750 TOPS),
-// 2048x4096x11008 238.3 -> 224.3, 1024x4096x4096 59.1 -> 56.5, 480x11008x4096
-// 90.1 -> 83.9, 480x1536x4096 19.8 -> 16.9, 333x4096x4096 31.6 -> 29.0,
-// 200x4096x11008 51.6 -> 48.7. Loading the pieces from their own byte address
-// (two past a dword for every other block), which needs no realignment, is
-// slower (269.5 against 261.0 and 35.9 against 29.0 us).
+// CU at 2.0 GHz: 163 cycles an item, 126 with the staging left out. The pieces and
+// the subtraction against block pairs (68 / 36 bytes) staged in a phase of their
+// own after each stage and the conversion v_cvt_f32_i32 (about 5 cycles), tile
+// choice included, us in one process: 2048x11008x4096 260.3 -> 250.3 (738 TOPS),
+// 2048x4096x11008 236.0 -> 230.3, 1024x4096x4096 60.6 -> 57.2, 480x11008x4096 86.0 ->
+// 77.9, 480x1536x4096 19.8 -> 16.8, 333x4096x4096 30.7 -> 26.6, 200x4096x11008 51.0 ->
+// 39.4. Loading the pieces from their own byte address (two past a dword for every
+// other block), which needs no realignment, is slower (2048x11008x4096 269.5 against
+// 261.0 us, 333x4096x4096 35.9 against 29.0).
 // Smaller problems use smaller tiles whose stage blocks are shared by several
 // K-waves (their partial sums are added through LDS at the end), so that one
 // workgroup keeps eight waves on its CU.
@@ -120,8 +119,8 @@ struct PieceRegs {
 // BM * nb * 34 < 2^32 for every k up to kMaxTiledK (mfma_supported declines
 // longer rows).
 // Consecutive lanes take consecutive pieces of a row, so a wave's load covers
-// whole runs of a few rows (a lane per block pair, as before, touched 32 rows
-// per load, and the address coalescer, not the VALU, set the staging's cost).
+// whole runs of a few rows (a lane per block pair would touch 32 rows per load,
+// and the address coalescer, not the VALU, would set the staging's cost).
 // Block j starts 34 j (18 j) bytes into the row: two bytes before a dword for
 // odd j, whose values are then dword-aligned, and on a dword for even j, whose
 // values sit two bytes off. Either way the piece is bytes [2, 18) or [4, 20) of
@@ -616,11 +615,11 @@ int64_t tiles_of(int64_t m, int64_t n, int64_t bm, int64_t bn) { return ((m + bm
 // fitted to 47 shapes with each tile forced (m 32..2048, n 100..14336, k 128..11008;
 // mostly within 8 %), us there: k = 4096, one tile per CU 32x32 11, 32x64 12.7,
 // 64x64 17.5, 128x64 27.5, 128x128 60, two 88, four of the 2-wave 64x64 55; two
-// rounds 64x64 33.6, 128x64 53.6. Against the tile counts that chose before, among
-// the plain 64x64, the 2-K-wave 32x32 and 64x64, and the 128x128 tiles:
-// 333x4096x4096 30.7 -> 27.9 us, 128x4096x4096 19.9 -> 13.5, 100x11008x4096 30.8 ->
-// 27.6, 333x1536x4096 20.0 -> 16.7, 200x4096x11008 51.8 -> 39.5, 480x4096x11008
-// 80.3 -> 68.8, 130x8000x1664 22.2 -> 15.7, 480x4096x1536 14.0 -> 13.4.
+// rounds 64x64 33.6, 128x64 53.6. Against a choice by tile counts among the plain
+// 64x64, the 2-K-wave 32x32 and 64x64, and the 128x128 tiles (with the staging of
+// that time): 333x4096x4096 30.7 -> 26.6 us, 100x11008x4096 34.2 -> 26.6, 333x1536x4096
+// 19.2 -> 17.0, 200x4096x11008 51.0 -> 39.4, 480x4096x11008 76.1 -> 69.0, 130x8000x1664
+// 20.7 -> 14.1, 480x4096x1536 14.0 -> 13.1.
 int64_t q4_0_tile_ns(int config, int64_t m, int64_t n, int64_t k, int cus) {
     auto rounds = [&](int64_t bm, int64_t bn) { return (tiles_of(m, n, bm, bn) + cus - 1) / cus; };
     auto padded = [&](int64_t unit) { return (k + unit - 1) / unit * unit; };

@@ -268,7 +268,7 @@ def bench_stats(args):
 
     rows = sorted(stats, key=lambda r: -float(r["TotalDurationNs"]))
     out = ["# bench.py kernel statistics (rocprofv3 --kernel-trace --stats)", "",
-           "Command (repository root on the GPU box), then the summary:", "```"]
+           "Commands (from the repository root):", "```"]
     out += list(args.command or [])
     out += ["```", "", "| kernel | calls | avg us | median us | min us | max us |", "|---|---|---|---|---|---|"]
     for r in rows:

@@ -31,7 +31,7 @@ def test_noalloc_rejects_shapes_beyond_the_scratch(pkg):
     # 3855 rows pass the size check. Null operands make a later host check end
     # the call (no device: the scratch lookup; a device: the quantizer's null
     # check), so nothing is launched on either kind of machine; fake non-null
-    # pointers would reach a kernel launch on a GPU box.
+    # pointers would reach a kernel launch on a machine with a GPU.
     rc = L.pfng_hip_compute_noalloc(0, None, None, None, 3855, 8, 4096, 0, None)
     assert rc != pkg.OK and "static scratch" not in pkg.last_error()
 
